@@ -400,6 +400,23 @@ PRNN_API int prnn_gru_head_backward_packed(const void* wx, const void* a_z, cons
                                            void* workspace, size_t workspace_bytes,
                                            void* stream);
 
+/* ---- residual of a trajectory --------------------------------------------
+ * *out (one float in device memory) = max over every step and channel of
+ * |f(H_{t-1}, x_t) - H_t| (NaN if any difference is), the quantity of the
+ * reference's residual gate (solvers/newton/__init__.py:582-636), each
+ * intermediate rounded to the storage type as its tensor ops round it.
+ * wx, r / a_*, h0 and states as in the solves (sLSTM states (B, T, 4, d), GRU
+ * states (B, T, d) with d = n_heads d_head, any d_head <= 128 unpadded);
+ * cu_seqlens (int32, n_seq + 1 entries, or NULL): a packed stream (B = 1)
+ * whose sequence q starts from h0 row q (zeros when h0 is NULL). */
+PRNN_API int prnn_slstm_residual(const void* wx, const void* r, const void* h0,
+                                 const void* states, float* out, int B, int T, int d, float eps,
+                                 int dtype, const int* cu_seqlens, int n_seq, void* stream);
+PRNN_API int prnn_gru_head_residual(const void* wx, const void* a_z, const void* a_r,
+                                    const void* a_n, const void* h0, const void* states,
+                                    float* out, int B, int T, int n_heads, int d_head, int dtype,
+                                    const int* cu_seqlens, int n_seq, void* stream);
+
 /* ---- T = 1 decode (serving loop) -----------------------------------------
  * One recurrent step.  state / out: (rows, 4, d) sLSTM or (rows, d) GRU;
  * wx: (B, 4d) / (B, 3d) for this step.  block_table: NULL (row b of state is

@@ -12,9 +12,9 @@ Control flow follows the reference (``solvers/newton/__init__.py:212-324,
   ``ParaSLSTM(mix='diag')`` and ``ParaGRU(mix='head')`` on a ROCm device;
   'eager' runs the reference's eager loop on the GPU (the sLSTM iterations in
   a kernel that rounds like the eager tensor ops);
-* after the solve the residual gate re-evaluates ``max |F|`` with the cell's
-  torch ``step`` and raises :class:`NewtonDivergenceError` above
-  ``residual_fail``.
+* after the solve the residual gate evaluates ``max |F|`` of the trajectory
+  (one kernel, rounded like the cell's tensor ops) and raises
+  :class:`NewtonDivergenceError` above ``residual_fail``.
 
 The Newton solve itself never runs on the CPU: inputs on another device, or
 backends this build does not provide ('triton', 'context_parallel'), raise
@@ -211,14 +211,32 @@ def _prepend_any(states: Tensor, h0: Tensor | None, cu_seqlens: Tensor | None) -
     return prepend_state_ragged(states, h0, cu_seqlens)
 
 
+def _max_residual(cell, wx, states, h0, cu_seqlens) -> float:
+    """max |f(H_{t-1}, x_t) - H_t| on the host: one kernel over ``wx = W_x(x)`` and
+    the states.  A cell whose step is not the library's own is evaluated by that."""
+    def own(base: type, *names: str) -> bool:
+        return isinstance(cell, base) and all(
+            getattr(getattr(cell, n), "__func__", None) is getattr(base, n) for n in names)
+
+    if own(ParaSLSTM, "step", "_acts", "_recurrent"):
+        return float(ops.slstm_residual(wx, cell.clipped_r(), h0, states, cu_seqlens,
+                                        eps=cell.eps))
+    if own(ParaGRU, "step", "_acts") and cell.mix == "head":
+        return float(ops.gru_head_residual(wx, *cell.clipped_a_head(), h0, states, cu_seqlens))
+    pred = cell.step(_prepend_any(states, h0, cu_seqlens), None, wx=wx)
+    return float((pred - states).abs().amax())
+
+
 def _fill_stats(cell, x, states, h0, config, *, iters, stats, history=(), known=None,
-                cu_seqlens=None) -> None:
-    """Residual gate (newton/__init__.py:582-636): one extra cell step over T."""
+                cu_seqlens=None, wx=None) -> None:
+    """Residual gate (newton/__init__.py:582-636): one extra cell step over T
+    (``wx``: the projection of ``x`` when the solve has it at hand)."""
     if stats is None and config.residual_fail is None:
         return
     if known is None:
-        pred = cell.step(_prepend_any(states, h0, cu_seqlens), x)
-        res = float((pred - states).detach().abs().amax())
+        with torch.no_grad():
+            res = _max_residual(cell, cell.W_x(x) if wx is None else wx, states.detach(), h0,
+                                cu_seqlens)
     else:
         res = known
     hist = tuple(history)
@@ -253,7 +271,7 @@ def _newton_solve(cell, x, config, *, h0, stats, wx=None, cu_seqlens=None,
                                                               cu_seqlens=cu_seqlens)
         if not torch.compiler.is_compiling():
             _fill_stats(cell, x, states, h0, config, iters=iters, stats=stats, history=history,
-                        known=last if current else None, cu_seqlens=cu_seqlens)
+                        known=last if current else None, cu_seqlens=cu_seqlens, wx=wx)
         return states
     if config.fused_early_exit and not torch.compiler.is_compiling():
         states, iters, history = _fused_early_exit(cell, wx, config, h0=h0,
@@ -272,7 +290,7 @@ def _newton_solve(cell, x, config, *, h0, stats, wx=None, cu_seqlens=None,
     )
     if not torch.compiler.is_compiling():
         _fill_stats(cell, x, states, gate_h0, config, iters=int(config.max_iters), stats=stats,
-                    cu_seqlens=cu_seqlens)
+                    cu_seqlens=cu_seqlens, wx=wx)
     return states
 
 
@@ -298,8 +316,7 @@ def _fused_early_exit(cell, wx, config, *, h0, cu_seqlens=None,
         work = ops.slstm_newton_step(wx, r, h0, work, omega=float(config.omega), eps=cell.eps,
                                      cu_seqlens=cu_seqlens, block_table=block_table)
         states = work.to(wx.dtype)
-        pred = cell.step(_prepend_any(states, gate_h0, cu_seqlens), None, wx=wx)
-        res = float((pred - states).abs().amax())
+        res = _max_residual(cell, wx, states, gate_h0, cu_seqlens)
         history.append(res)
         if res < atol:
             return states, it + 1, history
@@ -326,8 +343,7 @@ def _newton_eager(cell, wx, config, *, h0, cu_seqlens=None):
     history: list[float] = []
 
     def residual(states: Tensor) -> float:
-        pred = cell.step(_prepend_any(states, h0, cu_seqlens), None, wx=wx)
-        return float((pred - states).abs().amax())
+        return _max_residual(cell, wx, states, h0, cu_seqlens)
 
     if isinstance(cell, ParaSLSTM):
         r = cell.clipped_r()

@@ -472,9 +472,73 @@ def _(wx, r, h0, states, grad, cu_seqlens=None, *, eps):
     )
 
 
+def slstm_residual(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor,
+                   cu_seqlens: Tensor | None = None, *, eps: float) -> Tensor:
+    """``max |f(H_{t-1}, x_t) - H_t|`` of a trajectory as a one-element fp32
+    tensor (NaN if any difference is): the residual gate's reduction
+    (solvers/newton/__init__.py:582-636) in one pass over ``wx`` and ``states``,
+    rounded where the tensor ops of ``cell.step`` round.  Not a registered op:
+    its callers read the value on the host."""
+    batch, time, d_h = _slstm_shapes(wx, r)
+    code = _validate("slstm_residual", wx, r, h0, states)
+    if states.shape != (batch, time, 4, d_h):
+        raise ValueError(f"states shape {tuple(states.shape)} != {(batch, time, 4, d_h)}")
+    cs32, _, n_seq, h0 = _packed_args(cu_seqlens, None, wx, h0, d_h)
+    if cs32 is None:
+        h0 = _slstm_h0(h0, batch, d_h)
+    wx, r, states = wx.contiguous(), r.contiguous(), states.contiguous()
+    out = torch.empty(1, dtype=torch.float32, device=wx.device)
+    lib = _lib.load()
+    with torch.cuda.device(wx.device):
+        rc = lib.prnn_slstm_residual(
+            _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), batch, time, d_h, float(eps),
+            code, _ptr(cs32), n_seq, _stream(wx.device),
+        )
+    _lib.check(rc, "slstm_residual")
+    return out
+
+
 # ---------------------------------------------------------------------------
 # ParaGRU mix='head'
 # ---------------------------------------------------------------------------
+
+
+def gru_head_residual(wx: Tensor, a_z: Tensor, a_r: Tensor, a_n: Tensor, h0: Tensor | None,
+                      states: Tensor, cu_seqlens: Tensor | None = None) -> Tensor:
+    """``max |f(H_{t-1}, x_t) - H_t|`` of a head-GRU trajectory, as
+    :func:`slstm_residual`; any ``d_head <= 128``, heads as they are."""
+    n_heads, d_head, _ = a_z.shape
+    d_h = n_heads * d_head
+    batch, time, _ = wx.shape
+    code = _validate("gru_head_residual", wx, a_z, a_r, a_n, h0, states)
+    if wx.shape[-1] != 3 * d_h:
+        raise ValueError(f"wx last dim {wx.shape[-1]} != 3 * d_h={3 * d_h}")
+    if states.shape != (batch, time, d_h):
+        raise ValueError(f"states shape {tuple(states.shape)} != {(batch, time, d_h)}")
+    cs32, rows = None, batch
+    if cu_seqlens is not None:
+        from pararnn_amd.ragged import validate_cu_seqlens
+
+        if batch != 1:
+            raise ValueError(f"cu_seqlens packs wx with batch=1, got batch={batch}")
+        cs32 = validate_cu_seqlens(cu_seqlens, time, wx.device).to(torch.int32).contiguous()
+        rows = int(cs32.numel()) - 1
+    if h0 is not None:
+        if h0.shape != (rows, d_h):
+            raise ValueError(f"h0 shape {tuple(h0.shape)} != {(rows, d_h)}")
+        h0 = h0.contiguous()
+    wx, states = wx.contiguous(), states.contiguous()
+    a_z, a_r, a_n = a_z.contiguous(), a_r.contiguous(), a_n.contiguous()
+    out = torch.empty(1, dtype=torch.float32, device=wx.device)
+    lib = _lib.load()
+    with torch.cuda.device(wx.device):
+        rc = lib.prnn_gru_head_residual(
+            _ptr(wx), _ptr(a_z), _ptr(a_r), _ptr(a_n), _ptr(h0), _ptr(states), _ptr(out), batch,
+            time, n_heads, d_head, code, _ptr(cs32), 0 if cs32 is None else rows,
+            _stream(wx.device),
+        )
+    _lib.check(rc, "gru_head_residual")
+    return out
 
 
 @torch.library.custom_op("pararnn::newton_gru_head_fused", mutates_args=())
