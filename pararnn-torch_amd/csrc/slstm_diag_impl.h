@@ -67,18 +67,19 @@ static Shape newton_shape(int dtype, bool work_in) {
   return work_in ? tiles().newton_work : tiles().newton_guess;
 }
 
-// All Picard passes in one launch (bf16 storage); PRNN_SLSTM_PICARD_FUSED=0
-// selects one launch per pass instead (the fp32 path always does).
-static bool picard_fused(int dtype) {
+// All Picard passes in one launch; PRNN_SLSTM_PICARD_FUSED=0 selects one launch
+// per pass instead (rectangular batches).
+static bool picard_fused() {
   static const bool on = [] {
     const char* e = getenv("PRNN_SLSTM_PICARD_FUSED");
     return !(e && atoi(e) == 0);
   }();
-  return narrow(dtype) && on;
+  return on;
 }
 
 // Shapes of the fused launch: wx, the stage's pre-activations and h stay in
-// registers (4.5 per step).  PRNN_SLSTM_PICARD_TILES="<L>x<W>" for tuning.
+// registers (4.5 per step).  PRNN_SLSTM_PICARD_TILES="<L>x<W>" for tuning
+// (bf16).
 static const Shape kPicardShapes[] = {{24, 4}, {16, 4}, {20, 4}, {32, 4}};
 
 static Shape picard_shape(int dtype) {
@@ -92,6 +93,7 @@ static Shape picard_shape(int dtype) {
     }
     return r;
   }();
+  if (!narrow(dtype)) return kPicardF32;
   return deterministic() || dtype == PRNN_F16 ? kPicardDefault : s;
 }
 
@@ -106,20 +108,21 @@ static InitWs carve_init(void* base, int B, int T, int d, int P, int dtype, size
                          bool packed = false) {
   Carver cv(base);
   InitWs w;
-  // packed bf16 streams always take the single-launch warm start
-  w.fused = packed ? narrow(dtype) : picard_fused(dtype);
+  // packed streams always take the single-launch warm start
+  w.fused = packed || picard_fused();
   w.hbuf[0] = w.hbuf[1] = nullptr;
   w.hlast = nullptr;
   if (w.fused) {
     // Stage-indexed look-back words (a tile may run stages ahead of the
     // tiles that still read its earlier stages), cleared with the counters.
-    const Geo g = geometry(B, T, d, packed ? kPicardPacked : picard_shape(dtype));
+    const Geo g = geometry(B, T, d, packed ? picard_packed_shape(narrow(dtype))
+                                           : picard_shape(dtype));
     w.lb = carve_lookback(cv, g, 3 * (P + 1), 4 * (P + 1));
     w.hlast = static_cast<unsigned long long*>(
         cv.take(sizeof(unsigned long long) * static_cast<size_t>(P) * kCB * g.n_tiles));
     w.lb.clear_words = (cv.used - (reinterpret_cast<char*>(w.lb.counters) - cv.base)) / sizeof(int);
   } else {
-    const Geo g = geometry(B, T, d, packed ? kFrozenPackedF32 : frozen_shape(dtype));
+    const Geo g = geometry(B, T, d, frozen_shape(dtype));
     w.lb = carve_lookback(cv, g, 3, 4);
     const size_t hb = static_cast<size_t>(B) * T * d * elem_size(dtype);
     w.hbuf[0] = P >= 1 ? cv.take(hb) : nullptr;
@@ -250,15 +253,11 @@ static void launch_frozen(bool has_h, bool full_out, const TX* wx, const TX* r, 
 template <typename TX>
 static void frozen_pass(bool has_h, bool full_out, const TX* wx, const TX* r, const TX* h0,
                         const TX* src, TX* out_full, TX* out_h, int B, int T, int d, float eps,
-                        const Lookback& lb, int epoch, hipStream_t stream, const Packed& pk) {
+                        const Lookback& lb, int epoch, hipStream_t stream) {
 #define PRNN_LAUNCH(LL, WW, DD)                                                              \
   return launch_frozen<TX, LL, WW, DD>(has_h, full_out, wx, r, h0, src, out_full, out_h, B, T, \
                                        d, eps, lb, epoch, stream)
   if constexpr (sizeof(TX) == 4) {
-    // packed streams: fp32 only (bf16 takes the single-launch warm start)
-    if (pk.cu != nullptr)
-      return launch_frozen_packed(has_h, full_out, wx, r, h0, src, out_full, out_h, T, d, eps,
-                                  lb, epoch, stream, pk);
     if (deterministic()) PRNN_LAUNCH(kFrozenF32.L, kFrozenF32.W, true);
     PRNN_LAUNCH(kFrozenF32.L, kFrozenF32.W, false);
   } else {
@@ -284,10 +283,9 @@ static int run_init(const TX* wx, const TX* r, const TX* h0, TX* states, int B, 
                     int P, float eps, const InitWs& w, hipStream_t stream, const Packed& pk) {
   int rc = clear_status(w.lb, stream);
   if (rc != PRNN_OK) return rc;
-  if constexpr (sizeof(TX) == 2) {
-    if (w.fused) {
-      const Shape sh = pk.cu != nullptr ? kPicardDefault : picard_shape(dtype_code<TX>());
-      const Geo g = geometry(B, T, d, sh);
+  if (w.fused) {
+    const Shape sh = pk.cu != nullptr ? kPicardDefault : picard_shape(dtype_code<TX>());
+    const Geo g = geometry(B, T, d, sh);
 #define PRNN_LAUNCH(LL, WW, WPE, DD)                                                             \
   slstm_picard_fused_kernel<TX, LL, WW, WPE, DD, false>                                          \
       <<<dim3(g.n_tiles), dim3(64 * WW), 0, stream>>>(                                           \
@@ -295,22 +293,28 @@ static int run_init(const TX* wx, const TX* r, const TX* h0, TX* states, int B, 
           w.lb.incl, w.hlast, w.lb.tag_base, w.lb.spin(), Packed{nullptr, nullptr, 0})
 #define PRNN_SHAPE(LL, WW, WPE) \
   else if (sh.L == LL && sh.W == WW) PRNN_LAUNCH(LL, WW, WPE, false);
-      static_assert(kPicardDefault.L == 24 && kPicardDefault.W == 4, "default Picard shape");
-      timing_begin(stream);
-      if (pk.cu != nullptr)
-        launch_picard_packed(wx, r, h0, states, T, d, P, eps, w.lb, w.hlast, stream, pk);
-      else if (deterministic()) PRNN_LAUNCH(24, 4, 3, true);
+    static_assert(kPicardDefault.L == 24 && kPicardDefault.W == 4, "default Picard shape");
+    timing_begin(stream);
+    if (pk.cu != nullptr) {
+      launch_picard_packed(wx, r, h0, states, T, d, P, eps, w.lb, w.hlast, stream, pk);
+    } else if constexpr (sizeof(TX) == 4) {
+      if (deterministic())
+        PRNN_LAUNCH(kPicardF32.L, kPicardF32.W, 2, true);
+      else
+        PRNN_LAUNCH(kPicardF32.L, kPicardF32.W, 2, false);
+    } else {
+      if (deterministic()) PRNN_LAUNCH(24, 4, 3, true);
       else if constexpr (std::is_same<TX, f16>::value) PRNN_LAUNCH(24, 4, 3, false);
       PRNN_SHAPE(24, 4, 3)
       PRNN_SHAPE(16, 4, 4)
       PRNN_SHAPE(20, 4, 3)
       PRNN_SHAPE(32, 4, 2)
+    }
 #undef PRNN_SHAPE
 #undef PRNN_LAUNCH
-      timing_end(stream);
-      PRNN_HIP(hipGetLastError());
-      return PRNN_OK;
-    }
+    timing_end(stream);
+    PRNN_HIP(hipGetLastError());
+    return PRNN_OK;
   }
   // Pass 0: zero-hidden scan (pre = wx); passes 1..P freeze wx + R h_prev.
   timing_begin(stream);
@@ -319,7 +323,7 @@ static int run_init(const TX* wx, const TX* r, const TX* h0, TX* states, int B, 
     const bool last = p == P;
     TX* out_h = last ? nullptr : static_cast<TX*>(w.hbuf[p & 1]);
     frozen_pass<TX>(p > 0, last, wx, r, h0, src, last ? states : nullptr, out_h, B, T, d, eps,
-                    w.lb, p + 1, stream, pk);
+                    w.lb, p + 1, stream);
     PRNN_HIP(hipGetLastError());
   }
   timing_end(stream);

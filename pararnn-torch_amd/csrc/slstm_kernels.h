@@ -355,14 +355,18 @@ __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// (1b) all frozen-gate passes in one launch (16-bit storage: bf16 or fp16)
+// (1b) all frozen-gate passes in one launch
 // ---------------------------------------------------------------------------
 //
 // Pass p of the Picard warm start freezes the gates at wx + R * h_{p-1}[t-1]
 // (h_{p-1} the readout of pass p - 1, rounded to the storage type as the reference keeps
 // it in the tensor dtype).  Each tile runs stage p = 0 .. P over its own
-// steps with wx, the stage's pre-activations and its h trajectory held in
-// registers; only the last stage writes the state.  Stage p of a tile needs
+// steps with wx and its h trajectory held in registers; only the last stage
+// writes the state.  16-bit storage also holds the stage's pre-activations
+// (4.5 registers per step in all: their two roundings are a third of a
+// stage's arithmetic); fp32 holds wx and h (5 per step) and forms the
+// pre-activations again in pass 2, two operations per gate.  Stage p of a
+// tile needs
 //  * h_{p-1} at the step before the tile: the predecessor tile publishes the
 //    h of its last step after each stage (tagged word, stage-indexed);
 //  * the stage-p carry: a decoupled look-back on stage-indexed tagged words.
@@ -377,14 +381,15 @@ slstm_picard_fused_kernel(
     unsigned long long* __restrict__ incl, unsigned long long* __restrict__ hlast, int tag_base,
     Spin spin, Packed pk) {
   static_assert(L % 2 == 0, "h is packed two steps to a register");
-  static_assert(sizeof(TN) == 2, "16-bit storage");
-  using NT = Narrow<TN>;
+  constexpr bool F32 = sizeof(TN) == 4;
+  using NT = Narrow<typename std::conditional<F32, bf16, TN>::type>;  // 16-bit storage only
+  using XS = RowStash<TN>;
   // one predecessor per wave and look-back round: measured 4% faster than
   // two at config 3, with a quarter less polled traffic (22 against 29 B of
   // reads per element).  The deterministic walk, which must find an
   // inclusive carry inside its window, keeps two.
   constexpr int KP = DET ? 2 : 1;
-  constexpr uint32_t SZ = 2;
+  constexpr uint32_t SZ = sizeof(TN);
   __shared__ float s_agg[W][4][kCB];
   __shared__ float s_carry[W][3][kCB];
   __shared__ float s_hl[W][kCB];
@@ -435,17 +440,16 @@ slstm_picard_fused_kernel(
     hd_all = find_heads(pk, t0, n_steps);
   }
 
-  uint32_t xw[L][2], pre[L][2], hh[L / 2];
+  // pre and the packed h: 16-bit storage; hf (h of every step): fp32
+  uint32_t xw[L][XS::N], pre[F32 ? 1 : L][2], hh[F32 ? 1 : L / 2];
+  float hf[F32 ? L : 1];
+  if constexpr (F32) {
+#pragma unroll
+    for (int s = 0; s < L; ++s) hf[s] = 0.f;
+  }
   {
     const rsrc_t rx = make_rsrc(wx + first * row4 + c0, span4);
-    auto load = [&](int s) {
-      uint32_t v[4];
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        v[g] = __builtin_amdgcn_raw_buffer_load_b16(rx, voff, s * row4 * SZ + g * slot, 0);
-      xw[s][0] = v[0] | (v[1] << 16);
-      xw[s][1] = v[2] | (v[3] << 16);
-    };
+    auto load = [&](int s) { XS::load(rx, voff, s * row4 * SZ, slot, xw[s]); };
     if (n_steps == L) {
 #pragma unroll
       for (int s = 0; s < L; ++s) load(s);
@@ -456,7 +460,8 @@ slstm_picard_fused_kernel(
           load(s);
         } else {
           // steps past the end run unguarded in packed streams: defined zeros
-          xw[s][0] = xw[s][1] = 0u;
+#pragma unroll
+          for (int q = 0; q < XS::N; ++q) xw[s][q] = 0u;
         }
       }
     }
@@ -504,7 +509,18 @@ slstm_picard_fused_kernel(
     // Keep wx packed across stages: without this the compiler hoists the
     // 16-bit unpacking out of the stage loop and holds 4 floats per step.
 #pragma unroll
-    for (int s = 0; s < L; ++s) asm volatile("" : "+v"(xw[s][0]), "+v"(xw[s][1]));
+    for (int s = 0; s < L; ++s)
+#pragma unroll
+      for (int q = 0; q < XS::N; ++q) asm volatile("" : "+v"(xw[s][q]));
+    // fp32: the zero-hidden stage is the others with R = 0 and h = 0 (exact:
+    // x + 0 is x), one body for all
+    float rs[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) rs[g] = first_stage ? 0.f : r[g];
+    // wx + round(R h) of gate g of a step (fp32 storage)
+    auto pre32 = [&](int s, int g, float hp) {
+      return add_rn(__uint_as_float(xw[s][F32 ? g : 0]), mul_rn(rs[g], hp));
+    };
     // h_{p-1} at t0 - 1.
     float hp0 = 0.f;
     if (!first_stage) {
@@ -544,21 +560,32 @@ slstm_picard_fused_kernel(
     auto step1 = [&](int s, auto chk) {
       constexpr bool CHECK = decltype(chk)::value;
       const bool head = CHECK && hd.at(s);
-      if (first_stage) {
-        pre[s][0] = xw[s][0];
-        pre[s][1] = xw[s][1];
+      float zi, zf, zz;
+      if constexpr (F32) {
+        float hp = s == 0 ? hp0 : hf[s > 0 ? s - 1 : 0];
+        if (head) hp = first_stage ? 0.f : head_h(s);
+        zi = pre32(s, 0, hp);
+        zf = pre32(s, 1, hp);
+        zz = pre32(s, 2, hp);
       } else {
-        float hp =
-            s == 0 ? hp0 : ((s - 1) & 1 ? NT::hi(hh[(s - 1) >> 1]) : NT::lo(hh[(s - 1) >> 1]));
-        if (head) hp = head_h(s);
+        if (first_stage) {
+          pre[s][0] = xw[s][0];
+          pre[s][1] = xw[s][1];
+        } else {
+          float hp =
+              s == 0 ? hp0 : ((s - 1) & 1 ? NT::hi(hh[(s - 1) >> 1]) : NT::lo(hh[(s - 1) >> 1]));
+          if (head) hp = head_h(s);
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          // round(R h) and round(wx + round(R h)), two gates per conversion.
-          const uint32_t q = NT::pack(r[2 * k] * hp, r[2 * k + 1] * hp);
-          pre[s][k] = NT::pack(NT::lo(xw[s][k]) + NT::lo(q), NT::hi(xw[s][k]) + NT::hi(q));
+          for (int k = 0; k < 2; ++k) {
+            // round(R h) and round(wx + round(R h)), two gates per conversion.
+            const uint32_t q = NT::pack(r[2 * k] * hp, r[2 * k + 1] * hp);
+            pre[s][k] = NT::pack(NT::lo(xw[s][k]) + NT::lo(q), NT::hi(xw[s][k]) + NT::hi(q));
+          }
         }
+        zi = NT::lo(pre[s][0]);
+        zf = NT::hi(pre[s][0]);
+        zz = NT::lo(pre[s][1]);
       }
-      const float zi = NT::lo(pre[s][0]), zf = NT::hi(pre[s][0]), zz = NT::lo(pre[s][1]);
       // a head: the segment so far no longer matters (F = -inf), the state
       // restarts from the sequence's initial one
       if (head) {
@@ -597,10 +624,17 @@ slstm_picard_fused_kernel(
     s_agg[wave][1][lane] = a.M;
     s_agg[wave][2][lane] = a.N;
     s_agg[wave][3][lane] = a.C;
-    // Hold pre packed through the look-back: pass 2 unpacks it again rather
-    // than the compiler keeping four floats per step alive.
+    // Hold pre packed through the look-back: pass 2 unpacks it again (forms it
+    // again from wx and h in fp32) rather than the compiler keeping four floats
+    // per step alive.
 #pragma unroll
-    for (int s = 0; s < L; ++s) asm volatile("" : "+v"(pre[s][0]), "+v"(pre[s][1]));
+    for (int s = 0; s < L; ++s) {
+      if constexpr (F32) {
+        asm volatile("" : "+v"(xw[s][0]), "+v"(xw[s][1]), "+v"(xw[s][3]), "+v"(hf[s]));
+      } else {
+        asm volatile("" : "+v"(pre[s][0]), "+v"(pre[s][1]));
+      }
+    }
     __syncthreads();
 
     unsigned long long* incl_p = incl + p * stage_incl;
@@ -660,6 +694,7 @@ slstm_picard_fused_kernel(
     // last stage writes the state.
     float m = s_carry[wave][0][lane], n = s_carry[wave][1][lane], c = s_carry[wave][2][lane];
     float h_even = 0.f, h_last = 0.f;
+    float hp_old = hp0;  // fp32: h_{p-1} of the step before (hf holds h_p up to it)
     auto step2 = [&](int s, auto chk) {
       constexpr bool CHECK = decltype(chk)::value;
       if (CHECK && hd.at(s)) {
@@ -669,8 +704,19 @@ slstm_picard_fused_kernel(
         n = hs[1];
         m = hs[2];
       }
-      const float zi = NT::lo(pre[s][0]), zf = NT::hi(pre[s][0]);
-      const float zo = NT::hi(pre[s][1]);
+      float zi, zf, zo;
+      if constexpr (F32) {
+        float hp = hp_old;
+        if (CHECK && hd.at(s)) hp = first_stage ? 0.f : head_h(s);
+        zi = pre32(s, 0, hp);
+        zf = pre32(s, 1, hp);
+        zo = pre32(s, 3, hp);
+        hp_old = hf[s];
+      } else {
+        zi = NT::lo(pre[s][0]);
+        zf = NT::hi(pre[s][0]);
+        zo = NT::hi(pre[s][1]);
+      }
       fg_step_z(zi, zf, s_z[wave][s][lane], m, n, c);
       const float h = c * frcp((1.f + fexp(-zo)) * (n + eps));
       if constexpr (last_stage) {
@@ -679,6 +725,9 @@ slstm_picard_fused_kernel(
         stb<TN>(ro, voff, so + slot, n);
         stb<TN>(ro, voff, so + 2 * slot, m);
         stb<TN>(ro, voff, so + 3 * slot, h);
+      } else if constexpr (F32) {
+        hf[s] = h;
+        h_last = h;
       } else if (s & 1) {
         hh[s >> 1] = NT::pack(h_even, h);
         h_last = NT::hi(hh[s >> 1]);
@@ -1367,6 +1416,11 @@ constexpr Shape kNewtonGuessDefault{24, 4};
 constexpr Shape kNewtonWorkDefault{24, 4};
 constexpr Shape kNewtonF32{16, 8};
 constexpr Shape kPicardDefault{24, 4};
+// fp32, all six passes of P = 5 at d=512, B=8, T=16384: 0.86 ms (32x4, two waves
+// per SIMD, no spills) against 0.85 (20x4), 0.90 (16x4), 0.95 (12x4, 24x4) and
+// 2.18 ms as one launch per pass; at d=256, B=1, T=131072 0.58 against 0.63
+// (20x4) and 1.31 ms; at d=256, B=8, T=2048, P=3 84 against 93 and 142 us.
+constexpr Shape kPicardF32{32, 4};
 constexpr Shape kNewtonFusedDefault{20, 4};
 constexpr Shape kNewtonFusedF32{16, 4};
 
@@ -1374,7 +1428,10 @@ constexpr Shape kNewtonFusedF32{16, 4};
 // rectangular tile lengths (their packed bodies are one guarded, head-checked
 // loop: no spills); the single-iteration launches run shorter tiles.
 constexpr Shape kPicardPacked{24, 4};
-constexpr Shape kFrozenPackedF32{32, 4};
+// no spills at 28 steps; N=16019, d=860, 95 sequences: 0.36 ms against 0.375 (32
+// steps, 7 registers spilled) and 0.75 ms as one launch per pass
+constexpr Shape kPicardPackedF32{28, 4};
+inline Shape picard_packed_shape(bool narrow) { return narrow ? kPicardPacked : kPicardPackedF32; }
 constexpr Shape kNewtonFusedPacked{20, 4};
 constexpr Shape kNewtonFusedPackedF32{12, 4};
 constexpr Shape kNewtonPackedGuess{16, 4};
@@ -1398,10 +1455,6 @@ template <typename TN>
 void launch_picard_packed(const TN* wx, const TN* r, const TN* h0, TN* out, int T, int d,
                           int P, float eps, const Lookback& lb, unsigned long long* hlast,
                           hipStream_t stream, const Packed& pk);
-void launch_frozen_packed(bool has_h, bool full_out, const float* wx, const float* r,
-                          const float* h0, const float* src, float* out_full, float* out_h, int T,
-                          int d, float eps, const Lookback& lb, int epoch, hipStream_t stream,
-                          const Packed& pk);
 template <typename TX>
 void launch_newton_fused_packed(const TX* wx, const TX* r, const TX* h0, const TX* guess, TX* out,
                                 int T, int d, int K, float omega, float eps, const Lookback& lb,

@@ -15,10 +15,10 @@ template <typename TN>
 void launch_picard_packed(const TN* wx, const TN* r, const TN* h0, TN* out, int T, int d,
                           int P, float eps, const Lookback& lb, unsigned long long* hlast,
                           hipStream_t stream, const Packed& pk) {
-  constexpr Shape sh = kPicardPacked;
+  constexpr Shape sh = sizeof(TN) == 4 ? kPicardPackedF32 : kPicardPacked;
   const Geo g = geometry(1, T, d, sh);
 #define PRNN_LAUNCH(DD)                                                                         \
-  slstm_picard_fused_kernel<TN, sh.L, sh.W, 3, DD, true>                                   \
+  slstm_picard_fused_kernel<TN, sh.L, sh.W, sizeof(TN) == 4 ? 2 : 3, DD, true>             \
       <<<dim3(g.n_tiles), dim3(64 * sh.W), 0, stream>>>(                                        \
       wx, r, h0, out, 1, T, d, g.n_cb, g.n_tiles, P, eps, lb.counters + 1, lb.agg, lb.incl,   \
       hlast, lb.tag_base, lb.spin(), pk)
