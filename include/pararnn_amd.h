@@ -400,6 +400,30 @@ PRNN_API int prnn_gru_head_backward_packed(const void* wx, const void* a_z, cons
                                            void* workspace, size_t workspace_bytes,
                                            void* stream);
 
+/* ---- 64-wide head GRU as walks over time ---------------------------------
+ * The same solve and backward as prnn_gru_head_newton / _backward (and their
+ * packed forms when cu_seqlens is non-NULL; h0 then has a row per sequence),
+ * with one serial walk per (sequence, head) instead of the chunked scan: for
+ * calls whose sequences are many or short (the caller chooses).  The Newton
+ * workspace is laid out like the sLSTM ones (64 ticket counters, the status
+ * word that prnn_slstm_lookback_status reads, tagged words) and follows the
+ * same tag_base scheme; max_iters in [1, 64]. */
+PRNN_API size_t prnn_gru_head_walk_newton_workspace_size(int B, int T, int n_heads,
+                                                         int max_iters);
+PRNN_API int prnn_gru_head_walk_newton(const void* wx, const void* a_z, const void* a_r,
+                                       const void* a_n, const void* h0, void* out, int B, int T,
+                                       int n_heads, int max_iters, float omega, int dtype,
+                                       const int* cu_seqlens, int n_seq, void* workspace,
+                                       size_t workspace_bytes, int tag_base, void* stream);
+PRNN_API size_t prnn_gru_head_walk_backward_workspace_size(int B, int T, int n_heads,
+                                                           int packed);
+PRNN_API int prnn_gru_head_walk_backward(const void* wx, const void* a_z, const void* a_r,
+                                         const void* a_n, const void* h0, const void* states,
+                                         const void* grad, void* g_wx, float* g_a, float* g_h0,
+                                         int B, int T, int n_heads, int dtype,
+                                         const int* cu_seqlens, int n_seq, void* workspace,
+                                         size_t workspace_bytes, void* stream);
+
 /* ---- residual of a trajectory --------------------------------------------
  * *out (one float in device memory) = max over every step and channel of
  * |f(H_{t-1}, x_t) - H_t| (NaN if any difference is), the quantity of the

@@ -30,6 +30,8 @@
 #include "pararnn_amd.h"
 #include "prnn_host.h"
 
+#include "gru_walk.h"
+
 #include <algorithm>
 #include <type_traits>
 
@@ -1943,6 +1945,49 @@ static int run_bwd(const TX* wx, const TX* az, const TX* ar, const TX* an, const
   return PRNN_OK;
 }
 
+// The backward with the adjoint as walks over time (gru_walk.hip): no chunk
+// matrices and no carry scan, the walk forms the gates itself; then the same
+// dL/dA reduction, which reads r from the workspace.
+struct WalkBwdWs {
+  float* gates;
+  float* part;
+  int n_split, rows_per;
+  int* hq;
+};
+
+static WalkBwdWs carve_walk_bwd(void* base, int B, int T, int H, size_t* total, bool packed) {
+  const int n_chunks = (T + kChunk - 1) / kChunk;
+  Carver cv(base);
+  WalkBwdWs w;
+  w.gates = static_cast<float*>(
+      cv.take(sizeof(float) * static_cast<size_t>(B) * H * n_chunks * kChunk * 3 * DH));
+  ga_split(B, T, H, &w.n_split, &w.rows_per);
+  w.part = static_cast<float*>(
+      cv.take(sizeof(float) * static_cast<size_t>(w.n_split) * 3 * H * DH * DH));
+  w.hq = packed ? static_cast<int*>(cv.take(sizeof(int) * static_cast<size_t>(T))) : nullptr;
+  *total = cv.used;
+  return w;
+}
+
+template <typename TX, bool PK>
+static int run_walk_bwd(const TX* wx, const TX* az, const TX* ar, const TX* an, const TX* h0,
+                        const TX* states, const TX* grad, TX* g_wx, float* g_a, float* g_h0,
+                        int B, int T, int H, const WalkBwdWs& w, hipStream_t stream,
+                        const GPk& pk) {
+  const int n_chunks = (T + kChunk - 1) / kChunk;
+  gruk::launch_walk_reverse<TX>(wx, az, ar, an, h0, states, grad, g_wx, w.gates,
+                                h0 != nullptr ? g_h0 : nullptr, T, H, PK ? pk.n_seq : B, n_chunks,
+                                kChunk, PK ? pk.cu : nullptr, stream);
+  PRNN_HIP(hipGetLastError());
+  gru_ga_kernel<TX, PK><<<dim3(w.n_split * H), dim3(256), 0, stream>>>(
+      h0, states, w.gates, g_wx, B, T, H, n_chunks, w.n_split, w.rows_per, w.part, pk);
+  PRNN_HIP(hipGetLastError());
+  gru_ga_reduce_kernel<<<dim3((3 * H * DH * DH + 63) / 64), dim3(256), 0, stream>>>(
+      w.part, H, w.n_split, g_a);
+  PRNN_HIP(hipGetLastError());
+  return PRNN_OK;
+}
+
 static int check(int B, int T, int H, int dh, int K, int dtype) {
   if (B < 1 || T < 1 || H < 1)
     return fail(PRNN_ERR_VALUE, "B, T, n_heads must be >= 1, got B=%d T=%d n_heads=%d", B, T, H);
@@ -2122,4 +2167,54 @@ extern "C" PRNN_API int prnn_gru_head_backward_packed(const void* wx, const void
   if (!cu_seqlens) return fail(PRNN_ERR_VALUE, "cu_seqlens must be non-null");
   return head_backward_call(wx, a_z, a_r, a_n, h0, states, grad, g_wx, g_a, g_h0, 1, T, n_heads,
                             d_head, dtype, workspace, workspace_bytes, stream, cu_seqlens, n_seq);
+}
+
+extern "C" PRNN_API size_t prnn_gru_head_walk_backward_workspace_size(int B, int T, int n_heads,
+                                                                      int packed) {
+  if (gru::check(B, T, n_heads, gru::DH, 0, PRNN_F32) != PRNN_OK) return 0;
+  size_t total = 0;
+  gru::carve_walk_bwd(nullptr, B, T, n_heads, &total, packed != 0);
+  return total;
+}
+
+extern "C" PRNN_API int prnn_gru_head_walk_backward(const void* wx, const void* a_z,
+                                                    const void* a_r, const void* a_n,
+                                                    const void* h0, const void* states,
+                                                    const void* grad, void* g_wx, float* g_a,
+                                                    float* g_h0, int B, int T, int n_heads,
+                                                    int dtype, const int* cu_seqlens, int n_seq,
+                                                    void* workspace, size_t workspace_bytes,
+                                                    void* stream) {
+  int rc = gru::check(B, T, n_heads, gru::DH, 0, dtype);
+  if (rc != PRNN_OK) return rc;
+  const bool packed = cu_seqlens != nullptr;
+  if (packed && (B != 1 || n_seq < 1 || n_seq > T))
+    return fail(PRNN_ERR_VALUE, "a packed stream has B = 1 and n_seq in [1, T], got B=%d n_seq=%d",
+                B, n_seq);
+  if (!wx || !a_z || !a_r || !a_n || !states || !grad || !g_wx || !g_a || !workspace)
+    return fail(PRNN_ERR_VALUE,
+                "wx, a_z, a_r, a_n, states, grad, g_wx, g_a and workspace must be non-null");
+  size_t need = 0;
+  const gru::WalkBwdWs w = gru::carve_walk_bwd(workspace, B, T, n_heads, &need, packed);
+  if (workspace_bytes < need)
+    return fail(PRNN_ERR_VALUE, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const gru::GPk pk{cu_seqlens, w.hq, nullptr, n_seq};
+  if (packed) {
+    gru::gru_heads_kernel<<<dim3((T + 255) / 256), dim3(256), 0, s>>>(cu_seqlens, n_seq, T, w.hq);
+    PRNN_HIP(hipGetLastError());
+  }
+  return with_storage(dtype, [&](auto tag) {
+    using TX = decltype(tag);
+    const TX *x = static_cast<const TX*>(wx), *az = static_cast<const TX*>(a_z),
+             *ar = static_cast<const TX*>(a_r), *an = static_cast<const TX*>(a_n),
+             *h = static_cast<const TX*>(h0), *st = static_cast<const TX*>(states),
+             *gr = static_cast<const TX*>(grad);
+    TX* gw = static_cast<TX*>(g_wx);
+    if (packed)
+      return gru::run_walk_bwd<TX, true>(x, az, ar, an, h, st, gr, gw, g_a, g_h0, B, T, n_heads, w,
+                                         s, pk);
+    return gru::run_walk_bwd<TX, false>(x, az, ar, an, h, st, gr, gw, g_a, g_h0, B, T, n_heads, w,
+                                        s, pk);
+  });
 }

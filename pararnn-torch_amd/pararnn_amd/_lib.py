@@ -20,7 +20,7 @@ PRNN_OK = 0
 PRNN_ERR_VALUE = 1
 PRNN_ERR_TYPE = 2
 PRNN_ERR_RUNTIME = 3
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 # name -> (restype, argtypes); mirrors include/pararnn_amd.h
 _P = ctypes.c_void_p
@@ -95,6 +95,12 @@ SIGNATURES: dict[str, tuple] = {
     "prnn_gru_wide_newton_workspace_size": (_S, [_I, _I, _I, _I, _I]),
     "prnn_gru_wide_newton": (
         _I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P, _I, _P, _S, _I, _P]),
+    "prnn_gru_head_walk_newton_workspace_size": (_S, [_I, _I, _I, _I]),
+    "prnn_gru_head_walk_newton": (
+        _I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P, _I, _P, _S, _I, _P]),
+    "prnn_gru_head_walk_backward_workspace_size": (_S, [_I, _I, _I, _I]),
+    "prnn_gru_head_walk_backward": (
+        _I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _I, _P, _S, _P]),
     "prnn_slstm_residual": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _F, _I, _P, _I, _P]),
     "prnn_gru_head_residual": (
         _I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P]),

@@ -591,8 +591,50 @@ def newton_gru_head_fused(
     return _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega)
 
 
+def _walks(units: int, total: int, longest: int, iters: int) -> bool:
+    """Whether a head-GRU call (64-wide blocks) runs as walks over time
+    (``csrc/gru_walk.hip``) or as the chunked scan (``csrc/gru_head.hip``).
+
+    ``units`` walks (sequence x block) of ``total`` steps together, the longest
+    of ``longest``; ``iters`` Newton iterations, 0 for the eq. 2.6 backward.
+    Both sides' times in microseconds, fitted to MI355X measurements (fp32 and
+    bf16 alike) over 1-1024 units and 33-8192 steps:
+
+    * a walk step takes 0.41 us (adjoint 0.49), every iteration of a solve in
+      flight at once, 32 steps behind the last; beyond 256 walks the chip
+      advances about 440 of them per step time.
+    * the chunked scan costs per iteration its launches (80 us; adjoint 150)
+      and 3.0 ns per step and unit, 4.7 (adjoint 4.2) while it has too few
+      chunks for its matrix-core replays.
+
+    At 128 units of 1024 steps, K = 3: 0.61 against 1.63 ms; 8 units of 33 steps:
+    73 against 305 us; 32 units of 8192 steps: 3.32 against 2.43 ms, chunked.  A
+    walk has to be 15% ahead: the two meet at about 16 units of 1024 steps.
+
+    ``PARARNN_AMD_GRU_WALK=0`` / ``1`` forces one or the other; a tuning switch
+    of the chunked scan asks for that scan."""
+    force = os.environ.get("PARARNN_AMD_GRU_WALK")
+    if force in ("0", "1"):
+        return force == "1" and iters <= _WALK_MAX_ITERS
+    if iters > _WALK_MAX_ITERS or any(k in os.environ for k in _CHUNK_SWITCHES):
+        return False
+    n = max(1, iters)
+    replays = units * (-(-longest // 512)) >= 512
+    step = 0.41 if iters else 0.49
+    walk = 35 + step * (longest + 32 * (n - 1) + max(0, total * n - 256 * longest) / 440)
+    chunk = n * ((80 if iters else 150)
+                 + total * (0.003 if replays else 0.0047 if iters else 0.0042))
+    return 1.15 * walk < chunk
+
+
+_WALK_MAX_ITERS = 64  # PRNN_TAG_SPAN
+_CHUNK_SWITCHES = ("PRNN_GRU_REPLAY_MFMA", "PRNN_GRU_REV_MFMA", "PRNN_GRU_CARRY_SINGLE")
+
+
 def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
     """A rectangular batch, or (``cs``: checked int64 offsets) one packed stream."""
+    from pararnn_amd.ragged import longest_sequence
+
     n_heads, d_head, _ = a_z.shape
     d_h = n_heads * d_head
     batch, time, _ = wx.shape
@@ -611,6 +653,23 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
     h0 = None if h0 is None else hb.to_blocks(h0).contiguous()
     out = wx.new_empty(batch, time, hb.d_pad)
     lib = _lib.load()
+    cs32 = None if cs is None else cs.to(device=wx.device, dtype=torch.int32).contiguous()
+    nbytes = 0
+    if max_iters >= 1 and _walks(rows * hb.n_blocks, batch * time * hb.n_blocks,
+                                 time if cs is None else longest_sequence(cs, time), max_iters):
+        nbytes = lib.prnn_gru_head_walk_newton_workspace_size(batch, time, hb.n_blocks,
+                                                              int(max_iters))
+    if 0 < nbytes <= _wide_workspace_cap(wx.device):
+        with torch.cuda.device(wx.device):
+            ws, tag = _slstm_workspace(nbytes, wx.device)
+            rc = lib.prnn_gru_head_walk_newton(
+                _ptr(wx), _ptr(a_z), _ptr(a_r), _ptr(a_n), _ptr(h0), _ptr(out), batch, time,
+                hb.n_blocks, int(max_iters), float(omega), code, _ptr(cs32),
+                0 if cs is None else rows, _ptr(ws), ws.numel(), tag, _stream(wx.device),
+            )
+        _lib.check(rc, "newton_gru_head_fused")
+        _check_lookback(ws, "newton_gru_head_fused")
+        return hb.from_blocks(out)
     with torch.cuda.device(wx.device):
         if cs is None:
             nbytes = lib.prnn_gru_head_newton_workspace_size(batch, time, hb.n_blocks, 64,
@@ -622,7 +681,6 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
                 _stream(wx.device),
             )
         else:
-            cs32 = cs.to(device=wx.device, dtype=torch.int32).contiguous()
             nbytes = lib.prnn_gru_head_newton_packed_workspace_size(time, hb.n_blocks, 64,
                                                                     int(max_iters), code)
             ws = _workspace(nbytes, wx.device)
@@ -674,13 +732,15 @@ def gru_head_backward_fused(
         if t.shape != (batch, time, d_h):
             raise ValueError(f"{name} shape {tuple(t.shape)} != {(batch, time, d_h)}")
     cs32 = None
-    rows = batch
+    rows, longest = batch, time
     if cu_seqlens is not None:
-        from pararnn_amd.ragged import validate_cu_seqlens
+        from pararnn_amd.ragged import longest_sequence, validate_cu_seqlens
 
         if batch != 1:
             raise ValueError(f"cu_seqlens packs wx with batch=1, got batch={batch}")
-        cs32 = validate_cu_seqlens(cu_seqlens, time, wx.device).to(torch.int32).contiguous()
+        cs = validate_cu_seqlens(cu_seqlens, time, wx.device)
+        longest = longest_sequence(cs, time)
+        cs32 = cs.to(torch.int32).contiguous()
         rows = int(cs32.numel()) - 1
     if h0 is not None and h0.shape != (rows, d_h):
         raise ValueError(f"h0 shape {tuple(h0.shape)} != {(rows, d_h)}")
@@ -697,6 +757,18 @@ def gru_head_backward_fused(
     g_a = torch.empty(3, hb.n_blocks, 64, 64, dtype=torch.float32, device=wx.device)
     g_h0 = torch.zeros(rows, hb.d_pad, dtype=torch.float32, device=wx.device)
     lib = _lib.load()
+    if _walks(rows * hb.n_blocks, batch * time * hb.n_blocks, longest, 0):
+        with torch.cuda.device(wx.device):
+            nbytes = lib.prnn_gru_head_walk_backward_workspace_size(batch, time, hb.n_blocks,
+                                                                    int(cs32 is not None))
+            ws = _workspace(nbytes, wx.device)
+            rc = lib.prnn_gru_head_walk_backward(
+                _ptr(wx), _ptr(a_z), _ptr(a_r), _ptr(a_n), _ptr(h0), _ptr(states), _ptr(grad),
+                _ptr(g_wx), _ptr(g_a), _ptr(g_h0), batch, time, hb.n_blocks, code, _ptr(cs32),
+                0 if cs32 is None else rows, _ptr(ws), ws.numel(), _stream(wx.device),
+            )
+        _lib.check(rc, "gru_head_backward_fused")
+        return hb.from_blocks(g_wx, 3), hb.head_grads(g_a), hb.from_blocks(g_h0)
     with torch.cuda.device(wx.device):
         if cs32 is None:
             nbytes = lib.prnn_gru_head_backward_workspace_size(batch, time, hb.n_blocks, 64,

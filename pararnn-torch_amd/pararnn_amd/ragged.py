@@ -40,8 +40,9 @@ from torch import Tensor
 # The last offsets that passed the checks: weak references to the tensor given
 # and to the int64 one returned, each with its version counter (bumped by every
 # in-place write), so the solve and the ops it calls check one stream once,
-# with one device-to-host copy.
-_checked: tuple[tuple[tuple[weakref.ref, int], ...], int] | None = None
+# with one device-to-host copy.  With them the longest sequence's length, which
+# only decides how a stream is run (the kernels read the offsets themselves).
+_checked: tuple[tuple[tuple[weakref.ref, int], ...], int, int] | None = None
 
 
 def _known(t: Tensor, time: int) -> bool:
@@ -73,8 +74,18 @@ def validate_cu_seqlens(cu_seqlens: Tensor, time: int,
     if bool((host[1:] <= host[:-1]).any()):
         raise ValueError("cu_seqlens must be strictly increasing")
     _checked = (tuple((weakref.ref(t), t._version) for t in {id(cu_seqlens): cu_seqlens,
-                                                             id(cs): cs}.values()), int(time))
+                                                             id(cs): cs}.values()), int(time),
+                int((host[1:] - host[:-1]).max()))
     return cs
+
+
+def longest_sequence(cs: Tensor, time: int) -> int:
+    """Length of the longest sequence of checked offsets (no copy from the
+    device when they are the last ones checked)."""
+    c = _checked
+    if c is not None and _known(cs, time):
+        return c[2]
+    return int((cs[1:] - cs[:-1]).max())
 
 
 def segment_start_flags(cu_seqlens: Tensor, time: int, *, batch: int = 1) -> Tensor:

@@ -1,0 +1,50 @@
+"""Which head-GRU calls run as walks over time and which as the chunked scan
+(``ops._walks``), on the CPU."""
+
+import pytest
+
+from pararnn_amd import ops
+
+
+@pytest.fixture(autouse=True)
+def _plain(monkeypatch):
+    for k in ("PARARNN_AMD_GRU_WALK", *ops._CHUNK_SWITCHES):
+        monkeypatch.delenv(k, raising=False)
+
+
+@pytest.mark.parametrize("units,T,iters,walk", [
+    (1, 33, 3, True), (1, 128, 0, True), (8, 128, 3, True), (128, 1024, 3, True),
+    (512, 3000, 1, True), (512, 1024, 0, True), (32, 3000, 3, True),
+    (1, 8192, 3, False), (8, 4096, 3, False), (32, 8192, 3, False), (32, 32768, 3, False),
+    (64, 1024, 1, False), (64, 3000, 0, False), (1, 1024, 1, False)])
+def test_rectangular(units, T, iters, walk):
+    assert ops._walks(units, units * T, T, iters) is walk
+
+
+def test_one_long_sequence_among_short_ones_stays_chunked():
+    assert not ops._walks(64 * 8, (65536 + 63 * 1024) * 8, 65536, 3)
+    assert ops._walks(64 * 8, 64 * 1024 * 8, 1024, 3)
+
+
+def test_switches(monkeypatch):
+    assert not ops._walks(128, 128 * 128, 128, ops._WALK_MAX_ITERS + 1)
+    monkeypatch.setenv("PRNN_GRU_REPLAY_MFMA", "1")
+    assert not ops._walks(128, 128 * 128, 128, 3)
+    monkeypatch.setenv("PARARNN_AMD_GRU_WALK", "1")
+    assert ops._walks(1, 10**6, 10**6, 3)
+    assert not ops._walks(1, 16, 16, ops._WALK_MAX_ITERS + 1)
+    monkeypatch.setenv("PARARNN_AMD_GRU_WALK", "0")
+    assert not ops._walks(128, 128 * 128, 128, 3)
+
+
+def test_longest_sequence_follows_the_offsets():
+    import torch
+
+    from pararnn_amd.ragged import longest_sequence, validate_cu_seqlens
+
+    cs = torch.tensor([0, 3, 10, 12])
+    assert longest_sequence(validate_cu_seqlens(cs, 12), 12) == 7
+    cs[1] = 9
+    assert longest_sequence(validate_cu_seqlens(cs, 12), 12) == 9
+    other = torch.tensor([0, 5, 12])
+    assert longest_sequence(other, 12) == 7
