@@ -3,11 +3,11 @@
 //
 // A workgroup of 256 lanes owns one (sequence, head).  Its lanes play two
 // roles at once:
-//  * the walk, one step at a time: 32 channel pairs x 8 parts of the
-//    contraction index.  A lane keeps 8 entries of each of the three matrices
-//    for both channels of its pair and the eight parts of a pair, eight
-//    neighbouring lanes, meet through three DPP adds; LDS and a barrier only
-//    broadcast the two vectors the products read;
+//  * the walk, one step at a time: 16 groups of 4 channels x 16 parts of the
+//    contraction index.  A lane keeps 4 entries of each of the three matrices
+//    for the 4 channels of its group (a product reads one 16-byte LDS word) and
+//    the 16 parts of a group, a DPP row, meet through five DPP adds; LDS and a
+//    barrier only broadcast the two vectors the products read;
 //  * the gates of the next block of 16 steps, which do not depend on the walk,
 //    as fp32 MFMA products (16 steps x 64 channels x 64, wave w the columns
 //    16 w .. + 15), a few MFMA per walk step, in the shadow of the walk's LDS
@@ -30,8 +30,9 @@ constexpr int DH = 64;
 constexpr int kBlk = 16;          // steps per block
 constexpr int kThreads = 256;
 constexpr int kPad = DH + 4;      // LDS row stride of the MFMA operands (bank spread)
-constexpr int kEnt = 8;           // contraction entries per lane
+constexpr int kEnt = 4;           // contraction entries per lane
 constexpr int kParts = DH / kEnt;
+constexpr int kChan = 4;          // channels per lane group
 
 struct Lane {
   int c, part;         // walk: channel and part; `wr` lanes write the channel
@@ -43,7 +44,8 @@ __device__ __forceinline__ Lane lane_roles() {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   Lane o;
   o.part = lane & (kParts - 1);
-  o.c = 2 * (8 * wave + (lane >> 3)) + (o.part >> 2);
+  // channel 2 b1 + b0 of the group with (b1, b0) the part's upper bits (see dot_seg)
+  o.c = kChan * (4 * wave + (lane >> 4)) + (o.part >> 2);
   o.wr = (o.part & 3) == 0;
   o.li = lane & 15;
   o.g = lane >> 4;
@@ -52,42 +54,46 @@ __device__ __forceinline__ Lane lane_roles() {
   return o;
 }
 
-// Entries k in [8 part, 8 part + 8) of columns (COL) or rows c and c ^ 1 of a
-// head's (in, out) matrix: a[2 kk + i] for channel c ^ i.
+// Entries k in [4 part, 4 part + 4) of columns (COL) or rows c ^ i, i = 0 .. 3, of
+// a head's (in, out) matrix: a[4 kk + i].
+constexpr int kKeep = kChan * kEnt;
 template <typename TX, bool COL>
-__device__ __forceinline__ void load_pair(const TX* A, const Lane& l, float a[2 * kEnt]) {
+__device__ __forceinline__ void load_group(const TX* A, const Lane& l, float a[kKeep]) {
 #pragma unroll
   for (int kk = 0; kk < kEnt; ++kk)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kChan; ++i) {
       const int k = l.part * kEnt + kk, ch = l.c ^ i;
-      a[2 * kk + i] = ld(A + (COL ? k * DH + ch : ch * DH + k));
+      a[kChan * kk + i] = ld(A + (COL ? k * DH + ch : ch * DH + k));
     }
 }
 
-// The lane's 8 entries of a vector in LDS.
-struct Seg {
-  float4 x, y;
-};
+// The lane's entries of a vector in LDS.
+using Seg = float4;
 __device__ __forceinline__ Seg load_seg(const float* __restrict__ v, const Lane& l) {
-  const float4* p = reinterpret_cast<const float4*>(v + l.part * kEnt);
-  return Seg{p[0], p[1]};
+  return *reinterpret_cast<const float4*>(v + l.part * kEnt);
 }
 
-// sum_k a v for this lane's channel (every lane of the channel gets it).
-__device__ __forceinline__ float dot_seg(const float a[2 * kEnt], const Seg& v) {
-  const float e[kEnt] = {v.x.x, v.x.y, v.x.z, v.x.w, v.y.x, v.y.y, v.y.z, v.y.w};
-  float s0 = a[0] * e[0], s1 = a[1] * e[0];
+// sum_k a v for this lane's channel c.  s[i] is the lane's part of channel c ^ i;
+// parts p and 15 - p (row_mirror) differ in both upper bits, so what this lane
+// keeps, channels c and c ^ 1, are the other's s[3] and s[2]; then p and p ^ 7
+// (row_half_mirror), which keep c and c ^ 1; then the four parts of a quad.  The
+// halving costs no selects, as a lane's own channel is always s[0].
+__device__ __forceinline__ float dot_seg(const float a[kKeep], const Seg& v) {
+  const float e[kEnt] = {v.x, v.y, v.z, v.w};
+  float s[kChan];
 #pragma unroll
-  for (int k = 1; k < kEnt; ++k) {
-    s0 = fmaf(a[2 * k], e[k], s0);
-    s1 = fmaf(a[2 * k + 1], e[k], s1);
-  }
-  s0 += dppf<0xB1>(s0);
-  s1 += dppf<0xB1>(s1);
-  s0 += dppf<0x4E>(s0);
-  s1 += dppf<0x4E>(s1);
-  return s0 + dppf<0x141>(s1);
+  for (int i = 0; i < kChan; ++i) s[i] = a[i] * e[0];
+#pragma unroll
+  for (int k = 1; k < kEnt; ++k)
+#pragma unroll
+    for (int i = 0; i < kChan; ++i) s[i] = fmaf(a[kChan * k + i], e[k], s[i]);
+  s[1] += dppf<0x140>(s[2]);
+  s[0] += dppf<0x140>(s[3]);
+  s[0] += dppf<0x141>(s[1]);
+  s[0] += dppf<0xB1>(s[0]);
+  s[0] += dppf<0x4E>(s[0]);
+  return s[0];
 }
 
 // The gate products of one block, in slices.  Row i of the block's previous

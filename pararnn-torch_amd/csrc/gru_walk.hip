@@ -21,11 +21,12 @@
 // gruk_reverse_kernel: the eq. 2.6 adjoint at H*, one walk per (sequence, head)
 // from the last step down.
 //
-// Measured (fp32 / bf16 alike): 0.41 us per Newton step and 0.49 us per adjoint
+// Measured (fp32 / bf16 alike): 0.40 us per Newton step and 0.45 us per adjoint
 // step while every walk has a CU to itself, of which the gate products take
-// 0.05; 440 walks advance per step time when they are more (two workgroups per
-// CU).  K = 3, 128 walks of 1024 steps: 0.61 ms against 1.63 ms chunked, 512
-// walks: 1.55 against 4.6; adjoint, 512 walks of 1024: 0.85 against 1.85 ms.
+// 0.05 (8 parts of 2 channels instead of 16 of 4, twice the LDS words read per
+// product: 0.41 and 0.49); 440 walks advance per step time when they are more
+// (two workgroups per CU).  K = 3, 128 walks of 1024 steps: 0.61 ms against 1.63 ms chunked, 512
+// walks: 1.5 against 4.6; adjoint, 512 walks of 1024: 0.8 against 1.85 ms.
 // With the outputs stored step by step from the lanes that hold them instead
 // of whole rows per block a step took 0.43 and 0.55 us.
 //
@@ -83,10 +84,10 @@ __device__ __forceinline__ void newton_walk(
   const int d = H * DH;
   const size_t row_base = static_cast<size_t>(sp.row) * T;
   const size_t hcol = static_cast<size_t>(head) * DH;
-  float az[2 * kEnt], ar[2 * kEnt], an[2 * kEnt];
-  load_pair<TX, true>(a_z, l, az);
-  load_pair<TX, true>(a_r, l, ar);
-  load_pair<TX, true>(a_n, l, an);
+  float az[kKeep], ar[kKeep], an[kKeep];
+  load_group<TX, true>(a_z, l, az);
+  load_group<TX, true>(a_r, l, ar);
+  load_group<TX, true>(a_n, l, an);
   GateOps ops;
   ops.load(a_z, a_r, a_n, l);
 
@@ -230,13 +231,15 @@ __device__ __forceinline__ void newton_walk(
     const float base = ka.x * delta + (ka.y * dot_seg(az, dv) + ka.w);
     __syncthreads();
     const Seg wv = load_seg(sh.w, l);
+    // the next step's scalars, behind the vector in the LDS queue
+    const int sn = s + 1 < kBlk ? s + 1 : 0, bn = s + 1 < kBlk ? buf : buf ^ 1;
+    const float4 kan = sh.a[bn][sn][l.c];
+    const float2 kbn = sh.b[bn][sn][l.c];
     beside(2 * s + 1);
     delta = base + ka.z * dot_seg(an, wv);
     if (l.wr) sh.d[s][l.c] = delta;
-    __builtin_amdgcn_sched_barrier(0);
-    const int sn = s + 1 < kBlk ? s + 1 : 0, bn = s + 1 < kBlk ? buf : buf ^ 1;
-    ka = sh.a[bn][sn][l.c];
-    kb = sh.b[bn][sn][l.c];
+    ka = kan;
+    kb = kbn;
     __syncthreads();
   };
   int buf = 0;
@@ -345,10 +348,10 @@ gruk_reverse_kernel(const TX* __restrict__ wx, const TX* __restrict__ a_z,
   const int d = H * DH;
   const size_t row_base = static_cast<size_t>(sp.row) * T;
   const size_t hcol = static_cast<size_t>(head) * DH, hoff = hcol * DH;
-  float az[2 * kEnt], ar[2 * kEnt], an[2 * kEnt];
-  load_pair<TX, false>(a_z + hoff, l, az);
-  load_pair<TX, false>(a_r + hoff, l, ar);
-  load_pair<TX, false>(a_n + hoff, l, an);
+  float az[kKeep], ar[kKeep], an[kKeep];
+  load_group<TX, false>(a_z + hoff, l, az);
+  load_group<TX, false>(a_r + hoff, l, ar);
+  load_group<TX, false>(a_n + hoff, l, an);
   GateOps ops;
   ops.load(a_z + hoff, a_r + hoff, a_n + hoff, l);
 
@@ -431,14 +434,17 @@ gruk_reverse_kernel(const TX* __restrict__ wx, const TX* __restrict__ a_z,
     sh.g[0][s][l.c] = mu * ka.y;
     __syncthreads();
     const Seg nv = load_seg(sh.g[2][s], l), zv = load_seg(sh.g[0][s], l);
+    // the next step's scalars, behind the vectors in the LDS queue
+    const int sn = s + 1 < kBlk ? s + 1 : 0, bn = s + 1 < kBlk ? buf : buf ^ 1;
+    const float4 kan = sh.a[bn][sn][l.c];
+    const float2 kbn = sh.b[bn][sn][l.c];
     beside(2 * s);
     const float du = dot_seg(an, nv);
     sh.g[1][s][l.c] = du * kb.y;
     __builtin_amdgcn_sched_barrier(0);
     const float base = ka.x * mu + (kb.x * du + dot_seg(az, zv));
-    const int sn = s + 1 < kBlk ? s + 1 : 0, bn = s + 1 < kBlk ? buf : buf ^ 1;
-    ka = sh.a[bn][sn][l.c];
-    kb = sh.b[bn][sn][l.c];
+    ka = kan;
+    kb = kbn;
     __syncthreads();
     const Seg rv = load_seg(sh.g[1][s], l);
     beside(2 * s + 1);

@@ -600,7 +600,7 @@ def _walks(units: int, total: int, longest: int, iters: int) -> bool:
     Both sides' times in microseconds, fitted to MI355X measurements (fp32 and
     bf16 alike) over 1-1024 units and 33-8192 steps:
 
-    * a walk step takes 0.41 us (adjoint 0.49), every iteration of a solve in
+    * a walk step takes 0.40 us (adjoint 0.45), every iteration of a solve in
       flight at once, 32 steps behind the last; beyond 256 walks the chip
       advances about 440 of them per step time.
     * the chunked scan costs per iteration its launches (80 us; adjoint 150)
@@ -620,7 +620,7 @@ def _walks(units: int, total: int, longest: int, iters: int) -> bool:
         return False
     n = max(1, iters)
     replays = units * (-(-longest // 512)) >= 512
-    step = 0.41 if iters else 0.49
+    step = 0.40 if iters else 0.45
     walk = 35 + step * (longest + 32 * (n - 1) + max(0, total * n - 256 * longest) / 440)
     chunk = n * ((80 if iters else 150)
                  + total * (0.003 if replays else 0.0047 if iters else 0.0042))
