@@ -25,6 +25,8 @@ namespace gruk {
 using gruw::dppf;
 using gruw::floatx4;
 using gruw::lerp_t;
+using gruw::Scalars;
+using gruw::scalars;
 
 constexpr int DH = 64;
 constexpr int kBlk = 16;          // steps per block
@@ -170,16 +172,6 @@ __device__ __forceinline__ void gate_slice(int s, const GateOps& b, GateAcc& a,
     for (int v = 0; v < 4; ++v) a.n[v] = ftanh((a.n[v] + a.n1[v]) + to_f32(x[2][v]));
     done();
   }
-}
-
-// The scalars of a step and channel: J v = d1 v + d2 (A_z^T v) + d3 A_n^T (r v +
-// d5 (A_r^T v)) with d1 = 1 - z, d2 = (n - h) z (1 - z), d3 = z (1 - n^2),
-// d5 = h r (1 - r) (reference cells/para_gru.py:385-412).
-struct Scalars {
-  float d1, d2, d3, d5;
-};
-__device__ __forceinline__ Scalars scalars(float z, float r, float n, float h) {
-  return Scalars{1.f - z, (n - h) * z * (1.f - z), z * (1.f - n * n), h * r * (1.f - r)};
 }
 
 // The adjoint walk of every (sequence, block head); see gru_walk.hip.

@@ -16,10 +16,11 @@ namespace gruw {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int DW = 128;       // widest head
-constexpr int kParts = 8;     // parts of the contraction index
-constexpr int kKP = DW / kParts;  // contraction entries per lane (16)
-constexpr int kK = 2 * kKP;   // entries per lane and matrix: two channels (32)
-constexpr int kThreads = DW / 2 * kParts;
+constexpr int kParts = 16;    // parts of the contraction index
+constexpr int kKP = DW / kParts;  // contraction entries per lane (8)
+constexpr int kCh = 4;        // channels per lane group
+constexpr int kK = kCh * kKP;  // entries per lane and matrix (32)
+constexpr int kThreads = DW / kCh * kParts;
 // A broadcast vector sits in LDS in two halves of 64 entries, the second
 // shifted by four words (bank spread of the segments one wave reads).
 constexpr int kVec = DW + 4;
@@ -40,40 +41,38 @@ __device__ __forceinline__ Span span_of(int s, int T, const int* cu) {
   return Span{0, cu[s], cu[s + 1], s};
 }
 
-// Lane roles.  Lane l of wave w holds the channel pair 2 p, 2 p + 1 with
-// p = 8 w + l / 8, and the contraction entries k in [16 j, 16 j + 16) with
-// j = l % 8: its products read 16 entries of the broadcast vector and feed
-// two channels (half the LDS reads per multiply-add of one channel per
-// lane: the walks are bound by the LDS read rate).  After the reduction the
-// lanes j < 4 hold channel 2 p and the lanes j >= 4 channel 2 p + 1; j = 0
-// and j = 4 write it.
+// Lane roles.  The 16 lanes of a DPP row hold a group of four channels and the
+// 16 parts of the contraction index, entries k in [8 j, 8 j + 8) for part j: a
+// product reads 8 entries of the broadcast vector (two 16-byte LDS words) and
+// feeds four channels (the walks are bound by LDS reads and VALU issue; with 8
+// parts of 16 entries and two channels the one-launch solve took 0.72 us per
+// step).  After the reduction the lanes 4 q .. 4 q + 3 hold channel q of the
+// group; the first of them writes it.
 struct Role {
-  int pair, part, c;
+  int part, c;
   bool wr;
 };
 __device__ __forceinline__ Role role() {
   const int lane = threadIdx.x & 63;
   Role o;
   o.part = lane & (kParts - 1);
-  o.pair = (threadIdx.x >> 6) * 8 + (lane >> 3);
-  o.c = 2 * o.pair + (o.part >> 2);
+  o.c = kCh * ((threadIdx.x >> 6) * 4 + (lane >> 4)) + (o.part >> 2);
   o.wr = (o.part & 3) == 0;
   return o;
 }
 
-// Entries k in [16 j, 16 j + 16) of columns (COL) or rows 2 p, 2 p + 1 of a
-// head's A ((in, out) layout, d_head x d_head), zero outside the head, the
-// lane's own channel c first: a[2 kk + i] = A[k][ch_i] (COL) or A[ch_i][k]
-// with ch_0 = c and ch_1 the other channel of the pair.
+// Entries k in [8 j, 8 j + 8) of columns (COL) or rows c ^ i, i = 0 .. 3, of a
+// head's A ((in, out) layout, d_head x d_head), zero outside the head:
+// a[4 kk + i] = A[k][c ^ i] (COL) or A[c ^ i][k].
 template <typename TX, bool COL>
-__device__ __forceinline__ void load_pair(const TX* A, int dh, const Role& ro, float a[kK]) {
+__device__ __forceinline__ void load_group(const TX* A, int dh, const Role& ro, float a[kK]) {
 #pragma unroll
   for (int kk = 0; kk < kKP; ++kk)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kCh; ++i) {
       const int k = ro.part * kKP + kk, ch = ro.c ^ i;
       const bool in = ch < dh && k < dh;
-      a[2 * kk + i] =
+      a[kCh * kk + i] =
           in ? ld(A + (COL ? static_cast<size_t>(k) * dh + ch : static_cast<size_t>(ch) * dh + k))
              : 0.f;
     }
@@ -119,12 +118,16 @@ __device__ __forceinline__ Staged load_block(const float* __restrict__ z,
   return st;
 }
 
-__device__ __forceinline__ void store_block(float (*buf)[kS][DW], const Staged& st, int dh) {
+// Calls put(step, channel, z, r, n, hp, x) for the lane's four elements; dead
+// channels hold zeros.
+template <typename Put>
+__device__ __forceinline__ void take_block(const Staged& st, int dh, Put&& put) {
   const int cc = static_cast<int>(threadIdx.x) & (DW - 1);
+  const bool in = cc < dh;
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const int s = static_cast<int>(threadIdx.x) / DW + 4 * (j % 4);
-    buf[j / 4][s][cc] = cc < dh ? st.v[j] : 0.f;  // dead channels read zeros
+  for (int j = 0; j < 4; ++j) {
+    auto at = [&](int i) { return in ? st.v[4 * i + j] : 0.f; };
+    put(static_cast<int>(threadIdx.x) / DW + 4 * j, cc, at(0), at(1), at(2), at(3), at(4));
   }
 }
 
@@ -138,34 +141,51 @@ __device__ __forceinline__ float dppf(float v) {
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
-// sum_k A v for this lane's channel: the lane's 16 entries for both of its
-// pair's channels (one chain each: two chains per channel and the adds that
-// join them ran 2-3% slower), the sums over the eight parts of the
-// pair (quad_perm [1,0,3,2] and [2,3,0,1] within each quad for both
-// channels, then row_half_mirror between the two quads: each quad sends the
-// sum of the channel it does not keep, which the other quad keeps).  Every
-// lane of a channel ends with the same sum.
-__device__ __forceinline__ float dot_pair(const float a[kK], const float* __restrict__ v,
-                                          const Role& ro) {
-  const float* seg = v + slot(ro.part * kKP);
-  float s0 = 0.f, s1 = 0.f;
+// The lane's entries of a vector in LDS.
+struct Seg {
+  float4 x, y;
+};
+__device__ __forceinline__ Seg load_seg(const float* __restrict__ v, const Role& ro) {
+  const float4* p = reinterpret_cast<const float4*>(v + slot(ro.part * kKP));
+  return Seg{p[0], p[1]};
+}
+
+// sum_k A v for this lane's channel c (every lane of the channel gets it).
+// s[i] is the lane's part of channel c ^ i.  Parts p and 15 - p (row_mirror)
+// differ in both upper bits, so what this lane keeps, channels c and c ^ 1, are
+// the other's s[3] and s[2]; then p and p ^ 7 (row_half_mirror), which keep c and
+// c ^ 1; then the four parts of a quad.  The halving costs no selects, as a
+// lane's own channel is always s[0].
+__device__ __forceinline__ float dot_seg(const float a[kK], const Seg& v) {
+  const float e[kKP] = {v.x.x, v.x.y, v.x.z, v.x.w, v.y.x, v.y.y, v.y.z, v.y.w};
+  float s[kCh];
 #pragma unroll
-  for (int kk = 0; kk < kKP; kk += 4) {
-    const float4 x = *reinterpret_cast<const float4*>(seg + kk);
-    s0 = fmaf(a[2 * kk], x.x, s0);
-    s1 = fmaf(a[2 * kk + 1], x.x, s1);
-    s0 = fmaf(a[2 * kk + 2], x.y, s0);
-    s1 = fmaf(a[2 * kk + 3], x.y, s1);
-    s0 = fmaf(a[2 * kk + 4], x.z, s0);
-    s1 = fmaf(a[2 * kk + 5], x.z, s1);
-    s0 = fmaf(a[2 * kk + 6], x.w, s0);
-    s1 = fmaf(a[2 * kk + 7], x.w, s1);
-  }
-  s0 += dppf<0xB1>(s0);
-  s1 += dppf<0xB1>(s1);
-  s0 += dppf<0x4E>(s0);
-  s1 += dppf<0x4E>(s1);
-  return s0 + dppf<0x141>(s1);
+  for (int i = 0; i < kCh; ++i) s[i] = a[i] * e[0];
+#pragma unroll
+  for (int k = 1; k < kKP; ++k)
+#pragma unroll
+    for (int i = 0; i < kCh; ++i) s[i] = fmaf(a[kCh * k + i], e[k], s[i]);
+  s[1] += dppf<0x140>(s[2]);
+  s[0] += dppf<0x140>(s[3]);
+  s[0] += dppf<0x141>(s[1]);
+  s[0] += dppf<0xB1>(s[0]);
+  s[0] += dppf<0x4E>(s[0]);
+  return s[0];
+}
+__device__ __forceinline__ float dot(const float a[kK], const float* __restrict__ v,
+                                     const Role& ro) {
+  return dot_seg(a, load_seg(v, ro));
+}
+
+// The scalars of a step and channel, formed once when a block is staged (each
+// channel's lanes would repeat them): J v = d1 v + d2 (A_z^T v) + d3 A_n^T (r v +
+// d5 (A_r^T v)) with d1 = 1 - z, d2 = (n - h) z (1 - z), d3 = z (1 - n^2),
+// d5 = h r (1 - r) (reference cells/para_gru.py:385-412).
+struct Scalars {
+  float d1, d2, d3, d5;
+};
+__device__ __forceinline__ Scalars scalars(float z, float r, float n, float h) {
+  return Scalars{1.f - z, (n - h) * z * (1.f - z), z * (1.f - n * n), h * r * (1.f - r)};
 }
 
 static int check(int B, int T, int H, int dh, int dtype, const int* cu, int n_seq) {

@@ -15,14 +15,24 @@
 // with d2 = (n-h) z(1-z), d3 = z(1-n^2), d5 = h r(1-r) (reference
 // cells/para_gru.py:385-412), three 128-wide mat-vecs.
 //
-// Workgroup: 512 lanes = 64 channel pairs x 8 parts of the contraction index
-// (see Role): a lane keeps 16 entries of each A for both channels of its pair
-// in registers -- columns (forward: A^T products) or rows (adjoint: A
-// products) -- and the eight parts of a pair are eight neighbouring lanes, so
-// their partial sums meet through three DPP moves.  A step then needs LDS
-// and a barrier only to broadcast the two vectors the next products read:
-// two barriers per step.  fp32 throughout; channels >= d_head and entries
-// k >= d_head hold zeros.
+// Workgroup: 512 lanes = 32 channel groups x 16 parts of the contraction index
+// (see Role): a lane keeps 8 entries of each A for the four channels of its
+// group in registers -- columns (forward: A^T products) or rows (adjoint: A
+// products) -- and the sixteen parts of a group are a DPP row, so their partial
+// sums meet through four DPP steps.  A step then needs LDS and a barrier only to
+// broadcast the two vectors the next products read: two barriers per step.  fp32
+// throughout; channels >= d_head and entries k >= d_head hold zeros.
+//
+// What bounds a step: 3 128^2 FMA are 0.32 us of one CU's unpacked VALU; the rest
+// is the chain of the two broadcasts (LDS write, barrier, LDS read).  So a step
+// does nothing else: its scalars are formed when its block is staged, the next
+// step's are read behind the vector the current products read, and the rows of a
+// block are stored together at its end (a store at each step is one masked
+// dword per channel and waits in the step's chain).  B=4, T=2048, H=4,
+// d_head=128, fp32, per step: one iteration's walk 0.67 -> 0.61 us, three
+// iterations in one launch 0.78 -> 0.73, the adjoint op 0.79 -> 0.74.  Both walk
+// files are compiled with the iterative ILP scheduler (the walk 0.64 -> 0.59 us
+// per step, the adjoint 0.757 -> 0.727).
 #include "gru_wide.h"
 
 namespace prnn {
@@ -40,9 +50,12 @@ __global__ __launch_bounds__(kThreads) void gruw_walk_kernel(
     const float* __restrict__ hp, const float* __restrict__ hin, const TX* __restrict__ a_z,
     const TX* __restrict__ a_r, const TX* __restrict__ a_n, TOUT* __restrict__ out, int T,
     int H, int dh, float omega, const int* __restrict__ cu) {
-  __shared__ __attribute__((aligned(16))) float s_d[kVec];
+  __shared__ float4 s_a[2][kS][DW];  // d1, d2, d3, F
+  __shared__ float4 s_b[2][kS][DW];  // r, d5, H_t
+  // delta of a block's steps: the vector the next step reads, and at the end of
+  // the block what its rows are made of
+  __shared__ __attribute__((aligned(16))) float s_d[kS][kVec];
   __shared__ __attribute__((aligned(16))) float s_w[kVec];
-  __shared__ float s_in[2][kIn][kS][DW];
   const Role rl = role();
   const int c = rl.c;
   const int sc = slot(c);
@@ -50,54 +63,65 @@ __global__ __launch_bounds__(kThreads) void gruw_walk_kernel(
   const Span sp = span_of(blockIdx.x / H, T, cu);
   const size_t hoff = static_cast<size_t>(head) * dh * dh;
   float az[kK], ar[kK], an[kK];
-  load_pair<TX, true>(a_z + hoff, dh, rl, az);
-  load_pair<TX, true>(a_r + hoff, dh, rl, ar);
-  load_pair<TX, true>(a_n + hoff, dh, rl, an);
+  load_group<TX, true>(a_z + hoff, dh, rl, az);
+  load_group<TX, true>(a_r + hoff, dh, rl, ar);
+  load_group<TX, true>(a_n + hoff, dh, rl, an);
   const int d = H * dh;
-  const bool live = c < dh;
-  const size_t col = static_cast<size_t>(head) * dh + c;
-  if (rl.wr) s_d[sc] = 0.f;
+  if (rl.wr) s_d[kS - 1][sc] = 0.f;
   float delta = 0.f;
   if (sp.t0 >= sp.t1) return;
   const size_t row_base = static_cast<size_t>(sp.row) * T * d;
-  const rsrc_t ro = make_rsrc(out + row_base,
-                              static_cast<uint32_t>(static_cast<size_t>(T) * d * sizeof(TOUT)));
-  const uint32_t vo = (live && rl.wr) ? static_cast<uint32_t>(col * sizeof(TOUT)) : kOOB;
-  store_block(s_in[0], load_block(z, r, n, hp, hin, row_base, d, head, dh, sp.t0, 1, sp.t0,
-                                  sp.t1 - 1), dh);
+  auto load = [&](int t_first) {
+    return load_block(z, r, n, hp, hin, row_base, d, head, dh, t_first, 1, sp.t0, sp.t1 - 1);
+  };
+  auto take = [&](const Staged& st, int to) {
+    take_block(st, dh, [&](int s, int cc, float zt, float rt, float nt, float ht, float hv) {
+      const Scalars k = scalars(zt, rt, nt, ht);
+      s_a[to][s][cc] = float4{k.d1, k.d2, k.d3, lerp_t(ht, nt, zt) - hv};
+      s_b[to][s][cc] = float4{rt, k.d5, hv, 0.f};
+    });
+  };
+  const int fc = static_cast<int>(threadIdx.x) & (DW - 1), fs = static_cast<int>(threadIdx.x) / DW;
+  TOUT* o_col = out + row_base + static_cast<size_t>(head) * dh + fc;
+  auto flush = [&](int tb, int buf, int ns) {
+    if (fc >= dh) return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int s = fs + 4 * j;
+      if (s < ns)
+        st(o_col + static_cast<size_t>(tb + s) * d, s_b[buf][s][fc].z + omega * s_d[s][slot(fc)]);
+    }
+  };
+  take(load(sp.t0), 0);
   __syncthreads();
   int buf = 0;
   for (int tb = sp.t0; tb < sp.t1; tb += kS) {
     const bool more = tb + kS < sp.t1;
     Staged next;
-    if (more)
-      next = load_block(z, r, n, hp, hin, row_base, d, head, dh, tb + kS, 1, sp.t0, sp.t1 - 1);
+    if (more) next = load(tb + kS);
     const int ns = min(kS, sp.t1 - tb);
+    float4 ka = s_a[buf][0][c], kb = s_b[buf][0][c];
     for (int s = 0; s < ns; ++s) {
-      const int t = tb + s;
-      const float zt = s_in[buf][0][s][c], rt = s_in[buf][1][s][c], nt = s_in[buf][2][s][c];
-      const float ht = s_in[buf][3][s][c], hv = s_in[buf][4][s][c];
-      // A_r^T delta and A_z^T delta (delta_{t-1} broadcast in s_d)
-      const float sr = dot_pair(ar, s_d, rl);
-      const float sz = dot_pair(az, s_d, rl);
-      const float d5 = ht * rt * (1.f - rt);
-      if (rl.wr) s_w[sc] = rt * delta + d5 * sr;
+      // A_r^T delta and A_z^T delta (delta_{t-1}: the row before)
+      const Seg dv = load_seg(s_d[s > 0 ? s - 1 : kS - 1], rl);
+      const float w = kb.x * delta + kb.y * dot_seg(ar, dv);
+      if (rl.wr) s_w[sc] = w;
+      __builtin_amdgcn_sched_barrier(0);
+      const float base = ka.x * delta + (ka.y * dot_seg(az, dv) + ka.w);
       __syncthreads();
       // A_n^T (r delta + d5 A_r^T delta)
-      const float sn = dot_pair(an, s_w, rl);
-      const float d2 = (nt - ht) * zt * (1.f - zt);
-      const float d3 = zt * (1.f - nt * nt);
-      const float f = lerp_t(ht, nt, zt) - hv;
-      delta = (1.f - zt) * delta + d2 * sz + d3 * sn + f;
-      if (rl.wr) s_d[sc] = delta;
-      // a buffer store, dropped for lanes with the out-of-range offset
-      stb<TOUT>(ro, vo, static_cast<uint32_t>(t) * (d * sizeof(TOUT)), hv + omega * delta);
+      const Seg wv = load_seg(s_w, rl);
+      const int sn = min(s + 1, kS - 1);
+      const float4 kan = s_a[buf][sn][c], kbn = s_b[buf][sn][c];
+      delta = base + ka.z * dot_seg(an, wv);
+      if (rl.wr) s_d[s][sc] = delta;
+      ka = kan;
+      kb = kbn;
       __syncthreads();
     }
-    if (more) {
-      store_block(s_in[buf ^ 1], next, dh);
-      __syncthreads();
-    }
+    flush(tb, buf, ns);
+    if (more) take(next, buf ^ 1);
+    __syncthreads();
     buf ^= 1;
   }
 }
@@ -453,12 +477,22 @@ __device__ __forceinline__ void store_block_n(float (*x)[kSN][DW], float (*v)[kV
 constexpr int kGateWGs = 1;
 
 struct NewtonShared {
-  float x[2][3][kSN][DW];                               // wx (gates) or z, r, n (walks)
+  union {
+    struct {
+      float x[2][3][kSN][DW];                            // wx
+      __attribute__((aligned(16))) float hr[kSN][kVec];  // (h r) rows of a block
+    } g;                                                // gate workgroups
+    struct {
+      float4 a[2][kSN][DW];                             // d1, d2, d3, F
+      float2 b[2][kSN][DW];                             // r, d5
+      // delta of a block's steps: the vector the next step reads, and at the end
+      // of the block what its rows are made of
+      __attribute__((aligned(16))) float d[kSN][kVec];
+      __attribute__((aligned(16))) float w[kVec];        // r delta + d5 A_r^T delta
+    } w;                                                // walks
+  };
   __attribute__((aligned(16))) float v[2][kSN][kVec];   // H_{k-1}
   __attribute__((aligned(16))) float first[kVec];      // the sequence's initial state
-  __attribute__((aligned(16))) float d[kVec];          // walks: delta_{t-1}
-  __attribute__((aligned(16))) float w[kVec];          // walks: r delta + d5 A_r^T delta
-  __attribute__((aligned(16))) float hr[kSN][kVec];     // gates: (h r) rows of a block
 };
 
 // What both roles of a workgroup share.
@@ -498,7 +532,7 @@ __device__ __forceinline__ void newton_gates(NewtonShared& sh, const NewtonCtx& 
     StagedN<false, VT> st;
     load_block_n(st, src, at_of(tb), cx.d);
     await_block_n(st, src, at_of(tb), spin, gave_up);
-    store_block_n(sh.x[0], sh.v[0], st, cx.dh);
+    store_block_n(sh.g.x[0], sh.v[0], st, cx.dh);
   }
   __syncthreads();
   int buf = 0;
@@ -510,12 +544,13 @@ __device__ __forceinline__ void newton_gates(NewtonShared& sh, const NewtonCtx& 
     const int ns = min(kSN, sp.t1 - tb);
     auto gates_zr = [&](int s) {
       const float* hrow = tb + s == sp.t0 ? sh.first : sh.v[buf][s];
-      const float hz = dot_pair(az, hrow, rl);
-      const float hr = dot_pair(ar, hrow, rl);
-      const float z = fsigmoid(sh.x[buf][0][s][c] + hz);
-      const float r = fsigmoid(sh.x[buf][1][s][c] + hr);
+      const Seg hv = load_seg(hrow, rl);
+      const float hz = dot_seg(az, hv);
+      const float hr = dot_seg(ar, hv);
+      const float z = fsigmoid(sh.g.x[buf][0][s][c] + hz);
+      const float r = fsigmoid(sh.g.x[buf][1][s][c] + hr);
       if (rl.wr) {
-        sh.hr[s][sc] = hrow[sc] * r;
+        sh.g.hr[s][sc] = hrow[sc] * r;
         if (cx.live) {
           const size_t a = wide_at(cx.row_base, tb + s, cx.d, cx.col);
           st_tagged(gk + a, z, gtag);
@@ -524,8 +559,8 @@ __device__ __forceinline__ void newton_gates(NewtonShared& sh, const NewtonCtx& 
       }
     };
     auto gate_n = [&](int s) {
-      const float un = dot_pair(an, sh.hr[s], rl);
-      const float n = ftanh(sh.x[buf][2][s][c] + un);
+      const float un = dot(an, sh.g.hr[s], rl);
+      const float n = ftanh(sh.g.x[buf][2][s][c] + un);
       if (rl.wr && cx.live)
         st_tagged(gk + 2 * cx.btd + wide_at(cx.row_base, tb + s, cx.d, cx.col), n, gtag);
     };
@@ -544,7 +579,7 @@ __device__ __forceinline__ void newton_gates(NewtonShared& sh, const NewtonCtx& 
     }
     if (more) {
       await_block_n(next, src, at_of(tn), spin, gave_up);
-      store_block_n(sh.x[buf ^ 1], sh.v[buf ^ 1], next, cx.dh);
+      store_block_n(sh.g.x[buf ^ 1], sh.v[buf ^ 1], next, cx.dh);
     }
     // (h r) rows and the staging buffers are rewritten after this
     __syncthreads();
@@ -571,66 +606,95 @@ __device__ __forceinline__ void newton_walk(NewtonShared& sh, const NewtonCtx& c
     return BlockAt{cx.row_base, cx.d, ccol, t_first, 0, sp.t0, sp.t1 - 1};
   };
   bool gave_up = false;
+  // Block at t_first into buffer `to`: the iterate's rows, then (a barrier
+  // later, as a step's previous state is the row before) the scalars.
+  const int fs = static_cast<int>(threadIdx.x) / DW;
+  const int fc = static_cast<int>(threadIdx.x) & (DW - 1);
+  auto take = [&](const StagedN<true, VT>& st, int to, int t_first) {
+    const bool in = fc < cx.dh;
+    float v[kSP];
+#pragma unroll
+    for (int j = 0; j < kSP; ++j) {
+      if constexpr (VT)
+        v[j] = in ? word_val(st.v[j]) : 0.f;
+      else
+        v[j] = in ? st.v[j] : 0.f;
+      sh.v[to][fs + kRows * j][slot(fc)] = v[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSP; ++j) {
+      const int s = fs + kRows * j;
+      const float* hrow =
+          s > 0 ? sh.v[to][s - 1] : t_first == sp.t0 ? sh.first : sh.v[to ^ 1][kSN - 1];
+      const float z = in ? word_val(st.x[j]) : 0.f, r = in ? word_val(st.x[kSP + j]) : 0.f;
+      const float n = in ? word_val(st.x[2 * kSP + j]) : 0.f, hp = hrow[slot(fc)];
+      const Scalars k = scalars(z, r, n, hp);
+      sh.w.a[to][s][fc] = float4{k.d1, k.d2, k.d3, lerp_t(hp, n, z) - v[j]};
+      sh.w.b[to][s][fc] = float2{r, k.d5};
+    }
+  };
   {
     StagedN<true, VT> st;
     load_block_n(st, src, at_of(sp.t0), cx.d);
     await_block_n(st, src, at_of(sp.t0), spin, gave_up);
-    store_block_n(sh.x[0], sh.v[0], st, cx.dh);
+    take(st, 0, sp.t0);
   }
+  if (rl.wr) sh.w.d[kSN - 1][sc] = 0.f;
   __syncthreads();
   const bool last = cx.k == cx.K - 1;
   unsigned long long* dst = last ? nullptr : iters + cx.k * cx.btd;
   const int dst_tag = tag_base + 1 + cx.k;
-  const rsrc_t ro = make_rsrc(out + cx.row_base,
-                              static_cast<uint32_t>(static_cast<size_t>(cx.T) * cx.d * sizeof(TX)));
-  const uint32_t vo =
-      (last && cx.live && rl.wr) ? static_cast<uint32_t>(cx.col * sizeof(TX)) : kOOB;
+  // H_k = H_{k-1} + omega delta of a block's steps, whole rows at a time
+  auto flush = [&](int tb, int buf, int ns) {
+    if (fc >= cx.dh) return;
+#pragma unroll
+    for (int j = 0; j < kSP; ++j) {
+      const int s = fs + kRows * j;
+      if (s < ns) {
+        const float h = sh.v[buf][s][slot(fc)] + omega * sh.w.d[s][slot(fc)];
+        const size_t a = wide_at(cx.row_base, tb + s, cx.d, ccol);
+        if (last)
+          st(out + a, h);
+        else
+          st_tagged(dst + a, h, dst_tag);
+      }
+    }
+  };
   float delta = 0.f;
-  // this lane's word of the iterate at the current step (iterations before the last)
-  unsigned long long* dst_t =
-      dst == nullptr ? nullptr : dst + wide_at(cx.row_base, sp.t0, cx.d, cx.col);
   int buf = 0;
   for (int tb = sp.t0; tb < sp.t1; tb += kSN) {
     const bool more = tb + kSN < sp.t1;
     StagedN<true, VT> next;
     if (more) load_block_n(next, src, at_of(tb + kSN), cx.d);
     const int ns = min(kSN, sp.t1 - tb);
+    float4 ka = sh.w.a[buf][0][c];
+    float2 kb = sh.w.b[buf][0][c];
     for (int s = 0; s < ns; ++s) {
-      const int t = tb + s;
-      // previous state (the sequence's initial state, the other buffer's
-      // last row, or this block's previous row) and the iterate at t
-      const float* hrow =
-          s > 0 ? sh.v[buf][s - 1] : tb == sp.t0 ? sh.first : sh.v[buf ^ 1][kSN - 1];
-      const float hp = hrow[sc];
-      const float hin = sh.v[buf][s][sc];
-      const float z = sh.x[buf][0][s][c], r = sh.x[buf][1][s][c], n = sh.x[buf][2][s][c];
-      // A_r^T delta and A_z^T delta (delta_{t-1} broadcast in sh.d)
-      const float sr = dot_pair(ar, sh.d, rl);
-      const float sz = dot_pair(az, sh.d, rl);
-      const float d5 = hp * r * (1.f - r);
-      if (rl.wr) sh.w[sc] = r * delta + d5 * sr;
+      // A_r^T delta and A_z^T delta (delta_{t-1}: the row before)
+      const Seg dv = load_seg(sh.w.d[s > 0 ? s - 1 : kSN - 1], rl);
+      const float w = kb.x * delta + kb.y * dot_seg(ar, dv);
+      if (rl.wr) sh.w.w[sc] = w;
+      __builtin_amdgcn_sched_barrier(0);
+      const float base = ka.x * delta + (ka.y * dot_seg(az, dv) + ka.w);
       __syncthreads();
       // A_n^T (r delta + d5 A_r^T delta)
-      const float sn = dot_pair(an, sh.w, rl);
-      const float d2 = (n - hp) * z * (1.f - z);
-      const float d3 = z * (1.f - n * n);
-      const float f = lerp_t(hp, n, z) - hin;
-      delta = (1.f - z) * delta + d2 * sz + d3 * sn + f;
-      const float h_new = hin + omega * delta;
-      if (rl.wr) sh.d[sc] = delta;
-      if (dst != nullptr) {
-        if (cx.live && rl.wr) st_tagged(dst_t, h_new, dst_tag);
-        dst_t += cx.d;
-      } else {
-        stb<TX>(ro, vo, static_cast<uint32_t>(t) * (cx.d * sizeof(TX)), h_new);
-      }
+      const Seg wv = load_seg(sh.w.w, rl);
+      const int sn = min(s + 1, kSN - 1);
+      const float4 kan = sh.w.a[buf][sn][c];
+      const float2 kbn = sh.w.b[buf][sn][c];
+      delta = base + ka.z * dot_seg(an, wv);
+      if (rl.wr) sh.w.d[s][sc] = delta;
+      ka = kan;
+      kb = kbn;
       __syncthreads();
     }
+    flush(tb, buf, ns);
     if (more) {
       await_block_n(next, src, at_of(tb + kSN), spin, gave_up);
-      store_block_n(sh.x[buf ^ 1], sh.v[buf ^ 1], next, cx.dh);
-      __syncthreads();
+      take(next, buf ^ 1, tb + kSN);
     }
+    __syncthreads();
     buf ^= 1;
   }
 }
@@ -671,15 +735,13 @@ __global__ __launch_bounds__(kThreads) void gruw_newton_kernel(
   cx.row_base = static_cast<size_t>(cx.sp.row) * T * cx.d;
   const size_t hoff = static_cast<size_t>(cx.head) * dh * dh;
   float az[kK], ar[kK], an[kK];
-  load_pair<TX, true>(a_z + hoff, dh, cx.rl, az);
-  load_pair<TX, true>(a_r + hoff, dh, cx.rl, ar);
-  load_pair<TX, true>(a_n + hoff, dh, cx.rl, an);
-  // the sequence's initial state (h0 row or zeros) and delta_{t0-1} = 0
-  if (cx.rl.wr) {
+  load_group<TX, true>(a_z + hoff, dh, cx.rl, az);
+  load_group<TX, true>(a_r + hoff, dh, cx.rl, ar);
+  load_group<TX, true>(a_n + hoff, dh, cx.rl, an);
+  // the sequence's initial state (h0 row or zeros)
+  if (cx.rl.wr)
     sh.first[cx.sc] =
         (cx.live && h0 != nullptr) ? h0[static_cast<size_t>(cx.sp.seq) * cx.d + cx.col] : 0.f;
-    sh.d[cx.sc] = 0.f;
-  }
   if (cx.sp.t0 >= cx.sp.t1) return;
   // Iterations k and k + 2 share gate words: the gate workgroups of k + 2
   // reach block b only after the iterate of k + 1 covers it, i.e. after the

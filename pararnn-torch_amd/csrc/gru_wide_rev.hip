@@ -1,7 +1,6 @@
-// The eq. 2.6 adjoint walk of the wide-head tier (64 < d_head <= 128), in a
-// translation unit of its own: the build compiles it with the iterative ILP
-// scheduler, which shortens its per-step chain (the forward walks run slower
-// under that scheduler).
+// The eq. 2.6 adjoint walk of the wide-head tier (64 < d_head <= 128).  Laid out
+// like the forward walks (gru_wide.hip, which says what bounds a step and what it
+// measured).
 #include "gru_wide.h"
 
 namespace prnn {
@@ -20,10 +19,11 @@ __global__ __launch_bounds__(kThreads) void gruw_reverse_kernel(
     const float* __restrict__ hp, const TG* __restrict__ grad, const TX* __restrict__ a_z,
     const TX* __restrict__ a_r, const TX* __restrict__ a_n, float* __restrict__ g_wx,
     float* __restrict__ g_h0, int T, int H, int dh, const int* __restrict__ cu) {
-  __shared__ __attribute__((aligned(16))) float s_dz[kVec];
-  __shared__ __attribute__((aligned(16))) float s_dn[kVec];
-  __shared__ __attribute__((aligned(16))) float s_dr[kVec];
-  __shared__ float s_in[2][kIn][kS][DW];
+  __shared__ float4 s_a[2][kS][DW];  // d1, d2, d3, g
+  __shared__ float2 s_b[2][kS][DW];  // r, d5
+  // the pre-activation gradients of a block's steps: the vectors the products
+  // read, stored whole rows at a time at the end of the block
+  __shared__ __attribute__((aligned(16))) float s_g[3][kS][kVec];
   const Role rl = role();
   const int c = rl.c;
   const int sc = slot(c);
@@ -31,59 +31,77 @@ __global__ __launch_bounds__(kThreads) void gruw_reverse_kernel(
   const Span sp = span_of(blockIdx.x / H, T, cu);
   const size_t hoff = static_cast<size_t>(head) * dh * dh;
   float az[kK], ar[kK], an[kK];
-  load_pair<TX, false>(a_z + hoff, dh, rl, az);
-  load_pair<TX, false>(a_r + hoff, dh, rl, ar);
-  load_pair<TX, false>(a_n + hoff, dh, rl, an);
+  load_group<TX, false>(a_z + hoff, dh, rl, az);
+  load_group<TX, false>(a_r + hoff, dh, rl, ar);
+  load_group<TX, false>(a_n + hoff, dh, rl, an);
   const int d = H * dh;
   const bool live = c < dh;
   const size_t col = static_cast<size_t>(head) * dh + c;
   float nu = 0.f;
   if (sp.t0 >= sp.t1) return;
   const size_t row_base = static_cast<size_t>(sp.row) * T * d;
-  const rsrc_t rg = make_rsrc(g_wx + row_base * 3,
-                              static_cast<uint32_t>(static_cast<size_t>(T) * 3 * d * sizeof(float)));
-  const uint32_t vg = (live && rl.wr) ? static_cast<uint32_t>(col * sizeof(float)) : kOOB;
-  store_block(s_in[0], load_block(z, r, n, hp, grad, row_base, d, head, dh, sp.t1 - 1, -1,
-                                  sp.t0, sp.t1 - 1), dh);
+  auto load = [&](int t_first) {
+    return load_block(z, r, n, hp, grad, row_base, d, head, dh, t_first, -1, sp.t0, sp.t1 - 1);
+  };
+  auto take = [&](const Staged& st, int to) {
+    take_block(st, dh, [&](int s, int cc, float zt, float rt, float nt, float ht, float gt) {
+      const Scalars k = scalars(zt, rt, nt, ht);
+      s_a[to][s][cc] = float4{k.d1, k.d2, k.d3, gt};
+      s_b[to][s][cc] = float2{rt, k.d5};
+    });
+  };
+  // rows tb, tb - 1, ..., of dL/dwx from s_g
+  const int fc = static_cast<int>(threadIdx.x) & (DW - 1), fs = static_cast<int>(threadIdx.x) / DW;
+  float* g_col = g_wx + row_base * 3 + static_cast<size_t>(head) * dh + fc;
+  auto flush = [&](int tb, int ns) {
+    if (fc >= dh) return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int s = fs + 4 * j;
+      if (s < ns) {
+        float* p = g_col + static_cast<size_t>(tb - s) * 3 * d;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) p[static_cast<size_t>(q) * d] = s_g[q][s][slot(fc)];
+      }
+    }
+  };
+  take(load(sp.t1 - 1), 0);
   __syncthreads();
   int buf = 0;
   for (int tb = sp.t1 - 1; tb >= sp.t0; tb -= kS) {
     const bool more = tb - kS >= sp.t0;
     Staged next;
-    if (more)
-      next = load_block(z, r, n, hp, grad, row_base, d, head, dh, tb - kS, -1, sp.t0, sp.t1 - 1);
+    if (more) next = load(tb - kS);
     const int ns = min(kS, tb - sp.t0 + 1);
+    float4 ka = s_a[buf][0][c];
+    float2 kb = s_b[buf][0][c];
     for (int s = 0; s < ns; ++s) {
-      const int t = tb - s;
-      const float zt = s_in[buf][0][s][c], rt = s_in[buf][1][s][c], nt = s_in[buf][2][s][c];
-      const float ht = s_in[buf][3][s][c], g = s_in[buf][4][s][c];
-      const float mu = g + nu;
-      const float dz = mu * (nt - ht) * zt * (1.f - zt);
-      const float dn = mu * zt * (1.f - nt * nt);
+      const float mu = ka.w + nu;
       if (rl.wr) {
-        s_dz[sc] = dz;
-        s_dn[sc] = dn;
+        s_g[2][s][sc] = mu * ka.z;
+        s_g[0][s][sc] = mu * ka.y;
       }
       __syncthreads();
-      const float du = dot_pair(an, s_dn, rl);
-      const float azdz = dot_pair(az, s_dz, rl);
-      const float dr = du * ht * rt * (1.f - rt);
-      if (rl.wr) s_dr[sc] = dr;
+      const Seg nv = load_seg(s_g[2][s], rl), zv = load_seg(s_g[0][s], rl);
+      // the next step's scalars, behind the vectors in the LDS queue
+      const int sn = min(s + 1, kS - 1);
+      const float4 kan = s_a[buf][sn][c];
+      const float2 kbn = s_b[buf][sn][c];
+      const float du = dot_seg(an, nv);
+      const float dr = du * kb.y;
+      if (rl.wr) s_g[1][s][sc] = dr;
+      __builtin_amdgcn_sched_barrier(0);
+      const float base = ka.x * mu + (kb.x * du + dot_seg(az, zv));
+      ka = kan;
+      kb = kbn;
       __syncthreads();
-      const float ardr = dot_pair(ar, s_dr, rl);
-      nu = (1.f - zt) * mu + azdz + rt * du + ardr;
-      // buffer stores, dropped for the other lanes
-      const uint32_t so = static_cast<uint32_t>(t) * (3 * d * sizeof(float));
-      stb<float>(rg, vg, so, dz);
-      stb<float>(rg, vg, so + d * sizeof(float), dr);
-      stb<float>(rg, vg, so + 2 * d * sizeof(float), dn);
+      nu = base + dot(ar, s_g[1][s], rl);
     }
+    flush(tb, ns);
     // (the other staging buffer was last read a block ago, before this
     // block's barriers)
-    if (more) {
-      store_block(s_in[buf ^ 1], next, dh);
-      __syncthreads();
-    }
+    if (more) take(next, buf ^ 1);
+    __syncthreads();  // s_g is rewritten after this
     buf ^= 1;
   }
   // nu at the sequence's first step: dL/dh0 of its row
