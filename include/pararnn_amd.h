@@ -424,6 +424,25 @@ PRNN_API int prnn_gru_head_walk_backward(const void* wx, const void* a_z, const 
                                          const int* cu_seqlens, int n_seq, void* workspace,
                                          size_t workspace_bytes, void* stream);
 
+/* ---- narrow heads in 64-channel blocks -----------------------------------
+ * Moves arrays between a head GRU's own layout (n_heads heads of d_head <= 64
+ * channels) and the block layout of the kernels above: per = 64 / d_head heads
+ * at the first places of each of ceil(n_heads / per) blocks, zeros elsewhere.
+ * Up to 8 arrays per call, in one launch.  Channels (matrix = 0): rows of
+ * n_heads d_head values <-> rows of 64 n_blocks (an array of several gates has
+ * a row per gate).  Matrices (matrix = 1): rows stacks of (n_heads, d_head,
+ * d_head) <-> (n_blocks, 64, 64), block-diagonal.  to_blocks = 0: the way back
+ * (what lies outside the heads is left out).  No workspace. */
+typedef struct {
+  const void* src;
+  void* dst;
+  long long rows;
+  int matrix;
+  int elem_bytes; /* 2 or 4 */
+} prnn_block_move;
+PRNN_API int prnn_gru_head_blocks(const prnn_block_move* moves, int n_moves, int n_heads,
+                                  int d_head, int to_blocks, void* stream);
+
 /* ---- residual of a trajectory --------------------------------------------
  * *out (one float in device memory) = max over every step and channel of
  * |f(H_{t-1}, x_t) - H_t| (NaN if any difference is), the quantity of the

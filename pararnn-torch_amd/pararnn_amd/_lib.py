@@ -20,7 +20,14 @@ PRNN_OK = 0
 PRNN_ERR_VALUE = 1
 PRNN_ERR_TYPE = 2
 PRNN_ERR_RUNTIME = 3
-ABI_VERSION = 12
+ABI_VERSION = 13
+
+class BlockMove(ctypes.Structure):
+    """``prnn_block_move``."""
+
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("rows", ctypes.c_longlong),
+                ("matrix", ctypes.c_int), ("elem_bytes", ctypes.c_int)]
+
 
 # name -> (restype, argtypes); mirrors include/pararnn_amd.h
 _P = ctypes.c_void_p
@@ -101,6 +108,7 @@ SIGNATURES: dict[str, tuple] = {
     "prnn_gru_head_walk_backward_workspace_size": (_S, [_I, _I, _I, _I]),
     "prnn_gru_head_walk_backward": (
         _I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _I, _P, _S, _P]),
+    "prnn_gru_head_blocks": (_I, [ctypes.POINTER(BlockMove), _I, _I, _I, _I, _P]),
     "prnn_slstm_residual": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _F, _I, _P, _I, _P]),
     "prnn_gru_head_residual": (
         _I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P]),

@@ -17,6 +17,10 @@ scattered into a zero-padded block layout and gathered back; padded channels
 have zero inputs, zero weights and zero initial state, so they stay at zero
 (z = r = 1/2, n = 0 gives h' = h / 2) and never touch a real channel.
 
+The solves and their backward move everything a call needs in one launch
+(``ops._move_blocks``, ``csrc/gru_blocks.hip``); the tensor-op forms here serve the
+decode weights, which are laid out once, and the CPU.
+
 The reference handles ``d_head <= 64`` with a masked ``BLOCK_D`` tile
 (kernels/newton_gru_head.py:121-136).  Heads of 64 < d_head <= 128 take the
 wide tier instead (``ops._gru_head_wide``), not these blocks.
@@ -28,6 +32,8 @@ reference's masked tile keeps heads apart.  Finite inputs are unaffected.
 """
 
 from __future__ import annotations
+
+import functools
 
 import torch
 from torch import Tensor
@@ -48,18 +54,25 @@ class HeadBlocks:
         self.d_h = n_heads * d_head
         self.d_pad = self.n_blocks * BLOCK
         self.identity = BLOCK % d_head == 0 and n_heads % self.per == 0
-        if d_head != BLOCK:
-            # flat position in (n_blocks, 64, 64) of every (head, row, col)
-            h = torch.arange(n_heads, device=device).view(-1, 1, 1)
-            i = torch.arange(d_head, device=device).view(1, -1, 1)
-            j = torch.arange(d_head, device=device).view(1, 1, -1)
-            off = (h % self.per) * d_head
-            self.flat = ((h // self.per) * BLOCK * BLOCK + (off + i) * BLOCK + off + j).reshape(-1)
-        if not self.identity:
-            head = torch.arange(n_heads, device=device).repeat_interleave(d_head)
-            within = torch.arange(d_head, device=device).repeat(n_heads)
-            # padded channel of every real channel
-            self.chan = (head // self.per) * BLOCK + (head % self.per) * d_head + within
+        self.device = device
+
+    # The index maps of the tensor-op forms below, made when first used.
+
+    @functools.cached_property
+    def flat(self) -> Tensor:
+        """Flat position in ``(n_blocks, 64, 64)`` of every (head, row, col)."""
+        h = torch.arange(self.n_heads, device=self.device).view(-1, 1, 1)
+        i = torch.arange(self.d_head, device=self.device).view(1, -1, 1)
+        j = torch.arange(self.d_head, device=self.device).view(1, 1, -1)
+        off = (h % self.per) * self.d_head
+        return ((h // self.per) * BLOCK * BLOCK + (off + i) * BLOCK + off + j).reshape(-1)
+
+    @functools.cached_property
+    def chan(self) -> Tensor:
+        """Padded channel of every real channel."""
+        head = torch.arange(self.n_heads, device=self.device).repeat_interleave(self.d_head)
+        within = torch.arange(self.d_head, device=self.device).repeat(self.n_heads)
+        return (head // self.per) * BLOCK + (head % self.per) * self.d_head + within
 
     # -- weights ---------------------------------------------------------------
 

@@ -591,6 +591,61 @@ def newton_gru_head_fused(
     return _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega)
 
 
+def _to_blocks(hb: HeadBlocks, chans, mats) -> tuple[list, list]:
+    """``chans`` (``(..., gates * d_h)`` tensors or None, with their gates) and the
+    ``(H, d_head, d_head)`` matrices ``mats`` in the 64-channel blocks of the kernels,
+    contiguous: in one launch what the layout does not leave as it is."""
+    chans = [(None if t is None else t.contiguous(), g) for t, g in chans]
+    mats = [m.contiguous() for m in mats]
+    moves: list[tuple[Tensor, Tensor, int, int]] = []
+    if not hb.identity:
+        for k, (t, g) in enumerate(chans):
+            if t is not None:
+                out = t.new_empty(*t.shape[:-1], g * hb.d_pad)
+                moves.append((t, out, t.numel() // hb.d_h, 0))
+                chans[k] = (out, g)
+    if hb.d_head != 64:
+        block = mats[0].new_empty(len(mats), hb.n_blocks, 64, 64)
+        moves += [(m, out, 1, 1) for m, out in zip(mats, block)]
+        mats = list(block)
+    _move_blocks(hb, moves, 1)
+    return [t for t, _ in chans], mats
+
+
+def _from_blocks(hb: HeadBlocks, chans, mats=()) -> tuple[list, list]:
+    """The way back: ``(..., gates * d_pad)`` and ``(G, n_blocks, 64, 64)`` results
+    (contiguous) in the heads' own layout (of the matrices, the diagonal blocks; the
+    zeros around them are structural)."""
+    chans, mats = list(chans), list(mats)
+    moves: list[tuple[Tensor, Tensor, int, int]] = []
+    if not hb.identity:
+        for k, (t, g) in enumerate(chans):
+            out = t.new_empty(*t.shape[:-1], g * hb.d_h)
+            moves.append((t, out, t.numel() // hb.d_pad, 0))
+            chans[k] = (out, g)
+    if hb.d_head != 64:
+        for k, m in enumerate(mats):
+            out = m.new_empty(m.shape[0], hb.n_heads, hb.d_head, hb.d_head)
+            moves.append((m, out, m.shape[0], 1))
+            mats[k] = out
+    _move_blocks(hb, moves, 0)
+    return [t for t, _ in chans], mats
+
+
+def _move_blocks(hb: HeadBlocks, moves, to_blocks: int) -> None:
+    if not moves:
+        return
+    lib = _lib.load()
+    arr = (_lib.BlockMove * len(moves))(*(
+        _lib.BlockMove(src.data_ptr(), dst.data_ptr(), rows, matrix, src.element_size())
+        for src, dst, rows, matrix in moves))
+    dev = moves[0][0].device
+    with torch.cuda.device(dev):
+        rc = lib.prnn_gru_head_blocks(arr, len(moves), hb.n_heads, hb.d_head, to_blocks,
+                                      _stream(dev))
+    _lib.check(rc, "head blocks")
+
+
 def _walks(units: int, total: int, longest: int, iters: int) -> bool:
     """Whether a head-GRU call (64-wide blocks) runs as walks over time
     (``csrc/gru_walk.hip``) or as the chunked scan (``csrc/gru_head.hip``).
@@ -648,9 +703,7 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
         return _gru_head_wide(wx, a_z, a_r, a_n, h0, int(max_iters), float(omega), code, cs)
     # heads narrower than 64 run as block-diagonal 64 x 64 blocks
     hb = HeadBlocks(n_heads, d_head, wx.device)
-    wx = hb.to_blocks(wx, 3).contiguous()
-    a_z, a_r, a_n = (hb.matrices(a) for a in (a_z, a_r, a_n))
-    h0 = None if h0 is None else hb.to_blocks(h0).contiguous()
+    (wx, h0), (a_z, a_r, a_n) = _to_blocks(hb, [(wx, 3), (h0, 1)], [a_z, a_r, a_n])
     out = wx.new_empty(batch, time, hb.d_pad)
     lib = _lib.load()
     cs32 = None if cs is None else cs.to(device=wx.device, dtype=torch.int32).contiguous()
@@ -669,7 +722,7 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
             )
         _lib.check(rc, "newton_gru_head_fused")
         _check_lookback(ws, "newton_gru_head_fused")
-        return hb.from_blocks(out)
+        return _from_blocks(hb, [(out, 1)])[0][0]
     with torch.cuda.device(wx.device):
         if cs is None:
             nbytes = lib.prnn_gru_head_newton_workspace_size(batch, time, hb.n_blocks, 64,
@@ -690,7 +743,7 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
                 int(cs32.numel()) - 1, None, _ptr(ws), ws.numel(), _stream(wx.device),
             )
     _lib.check(rc, "newton_gru_head_fused")
-    return hb.from_blocks(out)
+    return _from_blocks(hb, [(out, 1)])[0][0]
 
 
 @newton_gru_head_fused.register_fake
@@ -748,11 +801,8 @@ def gru_head_backward_fused(
         return _gru_head_wide_backward(wx, a_z, a_r, a_n, h0, states, grad, code, cs32)
     # heads narrower than 64 run as block-diagonal 64 x 64 blocks
     hb = HeadBlocks(n_heads, d_head, wx.device)
-    wx = hb.to_blocks(wx, 3).contiguous()
-    states = hb.to_blocks(states).contiguous()
-    grad = hb.to_blocks(grad).contiguous()
-    a_z, a_r, a_n = (hb.matrices(a) for a in (a_z, a_r, a_n))
-    h0 = None if h0 is None else hb.to_blocks(h0).contiguous()
+    (wx, states, grad, h0), (a_z, a_r, a_n) = _to_blocks(
+        hb, [(wx, 3), (states, 1), (grad, 1), (h0, 1)], [a_z, a_r, a_n])
     g_wx = torch.empty_like(wx)
     g_a = torch.empty(3, hb.n_blocks, 64, 64, dtype=torch.float32, device=wx.device)
     g_h0 = torch.zeros(rows, hb.d_pad, dtype=torch.float32, device=wx.device)
@@ -768,7 +818,8 @@ def gru_head_backward_fused(
                 0 if cs32 is None else rows, _ptr(ws), ws.numel(), _stream(wx.device),
             )
         _lib.check(rc, "gru_head_backward_fused")
-        return hb.from_blocks(g_wx, 3), hb.head_grads(g_a), hb.from_blocks(g_h0)
+        (g_wx, g_h0), (g_a,) = _from_blocks(hb, [(g_wx, 3), (g_h0, 1)], [g_a])
+        return g_wx, g_a, g_h0
     with torch.cuda.device(wx.device):
         if cs32 is None:
             nbytes = lib.prnn_gru_head_backward_workspace_size(batch, time, hb.n_blocks, 64,
@@ -789,7 +840,8 @@ def gru_head_backward_fused(
                 rows, _ptr(ws), ws.numel(), _stream(wx.device),
             )
     _lib.check(rc, "gru_head_backward_fused")
-    return hb.from_blocks(g_wx, 3), hb.head_grads(g_a), hb.from_blocks(g_h0)
+    (g_wx, g_h0), (g_a,) = _from_blocks(hb, [(g_wx, 3), (g_h0, 1)], [g_a])
+    return g_wx, g_a, g_h0
 
 
 @gru_head_backward_fused.register_fake
