@@ -475,6 +475,21 @@ PRNN_API int prnn_gru_decode(const void* h, const void* wx, const void* a_z, con
                              const void* a_n, void* out, const int* block_table, int B, int d,
                              int n_heads, float cap, int has_cap, int dtype, void* stream);
 
+/* The same step from the cell's input: wx = x W^T + bias (x (B, d_in), W
+ * (gates * d, d_in) row major, bias (gates * d) or NULL, all of the storage
+ * type), rounded to that type as a GEMM's result is, in the step's own launch
+ * (the head GRU: a launch of its own, wx (B, 3d) its scratch; NULL otherwise).
+ * d_in times the element size a multiple of 16, x and W 16-byte aligned; out
+ * must not overlap x. */
+PRNN_API int prnn_slstm_decode_x(const void* state, const void* x, const void* w,
+                                 const void* bias, const void* r, void* out,
+                                 const int* block_table, int B, int d, int d_in, float eps,
+                                 float cap, int has_cap, int dtype, void* stream);
+PRNN_API int prnn_gru_decode_x(const void* h, const void* x, const void* w, const void* bias,
+                               const void* a_z, const void* a_r, const void* a_n, void* wx,
+                               void* out, const int* block_table, int B, int d, int d_in,
+                               int n_heads, float cap, int has_cap, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

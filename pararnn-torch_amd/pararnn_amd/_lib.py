@@ -20,7 +20,7 @@ PRNN_OK = 0
 PRNN_ERR_VALUE = 1
 PRNN_ERR_TYPE = 2
 PRNN_ERR_RUNTIME = 3
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 class BlockMove(ctypes.Structure):
     """``prnn_block_move``."""
@@ -114,6 +114,10 @@ SIGNATURES: dict[str, tuple] = {
         _I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P]),
     "prnn_slstm_decode": (_I, [_P, _P, _P, _P, _P, _I, _I, _F, _F, _I, _I, _P]),
     "prnn_gru_decode": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _I, _I, _P]),
+    "prnn_slstm_decode_x": (
+        _I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _F, _I, _I, _P]),
+    "prnn_gru_decode_x": (
+        _I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _I, _I, _P]),
 }
 
 _lock = threading.Lock()

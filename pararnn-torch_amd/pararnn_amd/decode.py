@@ -153,31 +153,95 @@ def _gru_recurrent(cell: ParaGRU) -> tuple[tuple[Tensor, Tensor, Tensor], int]:
     return hit[1], hit[2]
 
 
-def _launch(cell: nn.Module, kind: str, state: Tensor, gates: Tensor, tgt: _Target) -> None:
+def _projects(proj: nn.Module | None, rows: Tensor, d: int, gates: int, fused: bool,
+              out: Tensor) -> bool:
+    """Whether the step's kernel can do ``W_x(x)`` itself: a plain ``nn.Linear`` that
+    nothing watches or replaces (hooks, an instance ``forward``, a parametrization,
+    tensor subclasses, modes, autocast, tracing), on rows that it can read as they
+    are.  ``out`` must not overlap ``rows``: the projection is still being read when
+    the first channels of the next state are written."""
+    size = rows.element_size()
+    if type(proj) is not nn.Linear or not _small_step(rows.shape[0], d, rows.shape[1], size, fused):
+        return False
+    if (proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks
+            or proj._backward_pre_hooks or "forward" in proj.__dict__
+            or proj._compiled_call_impl is not None or nn.modules.module._has_any_global_hook()):
+        return False
+    w, bias = proj.weight, proj.bias
+    if (type(rows) is not Tensor or type(w) is not nn.Parameter
+            or type(bias) not in (nn.Parameter, type(None))
+            or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()):
+        return False
+    dtype, dev = rows.dtype, rows.device
+    if w.dtype != dtype or w.device != dev or w.shape != (gates * d, rows.shape[1]):
+        return False
+    if bias is not None and (bias.dtype != dtype or bias.device != dev
+                             or not bias.is_contiguous()):
+        return False
+    x0, w0, o0 = rows.data_ptr(), w.data_ptr(), out.data_ptr()
+    if (x0 | w0 | rows.shape[1] * size) % 16 or not rows.is_contiguous() or not w.is_contiguous():
+        return False
+    return (not rows.is_neg() and not w.is_neg() and rows.numel() > 0
+            and (x0 + rows.numel() * size <= o0 or o0 + out.numel() * out.element_size() <= x0))
+
+
+def _small_step(rows: int, d: int, d_in: int, size: int, fused: bool) -> bool:
+    """Whether a step's projection runs in the step's kernel or as a library GEMM.
+
+    A live step is bound by the host: the GEMM's dispatch is about 20 of its 38 us,
+    and one launch of the kernel takes 19 whatever the size.  Replayed from a
+    captured graph only the GPU counts, so the line lies where the kernel is the
+    faster one there too (us of the whole step, library / kernel, sLSTM):
+
+    * 16 bits: (rows, d = d_in) = (1, 1024) 8.3 / 4.2, (64, 1024) 8.6 / 7.1,
+      (16, 2048) 11.0 / 10.2; (32, 2048) 11.5 / 13.0.  Head GRU (64, 1024) 13.4 / 13.4.
+    * float32, whose matrix rate is an eighth: (1, 1024) 9.6 / 5.3, (16, 1024)
+      8.1 / 6.7, (64, 512) 9.8 / 6.5; (64, 1024) 11.5 / 12.3, (4, 2048) 15.5 / 15.7.
+      A head GRU's projection is a launch of its own: (64, 512) 13.7 / 12.0,
+      (16, 1024) 11.5 / 12.1.
+    """
+    if size == 2:
+        return rows * d * d_in <= 1 << 26
+    return rows * d * d_in <= 1 << 24 and d_in <= (1024 if fused else 512)
+
+
+def _launch(cell: nn.Module, kind: str, state: Tensor, gates: Tensor, tgt: _Target,
+            proj: nn.Linear | None = None) -> None:
+    """One step from the projected input ``gates``, or with ``proj`` from its input."""
     lib = _lib.load()
     d = int(cell.d_h)
     cap = cell.max_recurrent_norm
     clamp = (0.0, 0) if cap is None else (float(cap), 1)
     table = None if tgt.table is None else _ptr(tgt.table)
+    # the leading operands of either entry
+    src = (_ptr(gates),) if proj is None else (_ptr(gates), _ptr(proj.weight), _ptr(proj.bias))
+    d_in = () if proj is None else (int(gates.shape[1]),)
     if kind == "slstm":
-        if gates.shape[-1] != 4 * d:
+        if proj is None and gates.shape[-1] != 4 * d:
             raise ValueError(f"ParaSLSTM wx last dim {gates.shape[-1]} != 4 * d_h={4 * d}")
         r = cell.R if cell.R.is_contiguous() else cell.R.contiguous()
         code = _validate("decode_slstm", state, gates, r, tgt.out)
         with torch.cuda.device(state.device):
-            rc = lib.prnn_slstm_decode(_ptr(state), _ptr(gates), _ptr(r), _ptr(tgt.out), table,
-                                       tgt.rows, d, float(cell.eps), *clamp, code,
-                                       _stream(state.device))
+            entry = lib.prnn_slstm_decode if proj is None else lib.prnn_slstm_decode_x
+            rc = entry(_ptr(state), *src, _ptr(r), _ptr(tgt.out), table, tgt.rows, d, *d_in,
+                       float(cell.eps), *clamp, code, _stream(state.device))
         _lib.check(rc, "decode_slstm")
         return
-    if gates.shape[-1] != 3 * d:
+    if proj is None and gates.shape[-1] != 3 * d:
         raise ValueError(f"ParaGRU wx last dim {gates.shape[-1]} != 3 * d_h={3 * d}")
     (a_z, a_r, a_n), blocks = _gru_recurrent(cell)
     code = _validate("decode_gru", state, gates, a_z, a_r, a_n, tgt.out)
+    mats = (_ptr(a_z), _ptr(a_r), _ptr(a_n))
     with torch.cuda.device(state.device):
-        rc = lib.prnn_gru_decode(_ptr(state), _ptr(gates), _ptr(a_z), _ptr(a_r), _ptr(a_n),
-                                 _ptr(tgt.out), table, tgt.rows, d, blocks, *clamp, code,
-                                 _stream(state.device))
+        if proj is None:
+            rc = lib.prnn_gru_decode(_ptr(state), *src, *mats, _ptr(tgt.out), table, tgt.rows, d,
+                                     blocks, *clamp, code, _stream(state.device))
+        else:
+            wx = None if blocks == 0 else gates.new_empty(tgt.rows, 3 * d)
+            rc = lib.prnn_gru_decode_x(_ptr(state), *src, *mats, _ptr(wx), _ptr(tgt.out), table,
+                                       tgt.rows, d, *d_in, blocks, *clamp, code,
+                                       _stream(state.device))
     _lib.check(rc, "decode_gru")
 
 
@@ -200,12 +264,23 @@ def decode_step(cell: nn.Module, state: Tensor, x: Tensor | None = None, *,
         nxt = cell.step(state, x) if wx is None else cell.step(state, x, wx=wx)
         return nxt if out is None else out.copy_(nxt)
     capturing = torch.cuda.is_current_stream_capturing()
-    gates = _one_step(decode_wx(cell, x) if wx is None else wx, "wx")
+    proj = None
+    if wx is None:
+        gates = _one_step(x, "x")
+        linear = getattr(cell, "W_x", None)
+        dest = out if out is not None else state
+        if _projects(linear, gates, int(cell.d_h), 4 if kind == "slstm" else 3,
+                     cell.mix == "diag", dest):
+            proj = linear
+        else:
+            gates = decode_wx(cell, x)
+    else:
+        gates = _one_step(wx, "wx")
     gates = _laid_out(gates, "wx", capturing)
     state = _laid_out(state, "state", capturing)
     tgt = _target(state, out, block_table, capturing)
     if gates.shape[0] != tgt.rows:
         raise ValueError(f"decode_step wx has {gates.shape[0]} rows, the step advances "
                          f"{tgt.rows}")
-    _launch(cell, kind, state, gates, tgt)
+    _launch(cell, kind, state, gates, tgt, proj)
     return tgt.out
