@@ -868,7 +868,7 @@ __global__ __launch_bounds__(64 * W) void slstm_newton_kernel(
         }
       } else {
         CellJ J = cell_jac(prev, x, r, eps);
-        if (head) J.f = J.cm = J.ch = J.nm = J.nh = J.al = J.mh = J.inv = J.g = 0.f;
+        if (head) J.f = J.cm = J.ch = J.nm = J.nh = J.al = J.mh = J.inv = J.dn = J.g = 0.f;
         const float F[4] = {J.pc - hv[0], J.pn - hv[1], J.pm - hv[2], J.ph - hv[3]};
         jmv_affine(J, F, a.b);
 #pragma unroll
@@ -994,7 +994,10 @@ __global__ __launch_bounds__(64 * W) void slstm_newton_kernel(
           stb<TOUT>(ro, vo, so + k * d * sizeof(TOUT),
                     add_rn(hv[k], mul_rn(omega, round_to<TX>(dl[k]))));
       } else {
-        cell_delta<false>(prev, x, r, eps, 0.f, hv, dl);
+        float pv[4], jv[4];
+        cell_jvp(prev, x, r, eps, dl, pv, jv);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) dl[k] = jv[k] + (pv[k] - hv[k]);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
           stb<TOUT>(ro, vo, so + k * d * sizeof(TOUT), hv[k] + omega * dl[k]);
@@ -1354,9 +1357,11 @@ slstm_newton_fused_kernel(
         XS::get(xs[s], x);
 #pragma unroll
         for (int j = 0; j < 4; ++j) hv[j] = hf[s][j];
-        cell_delta<true>(prev, x, r, eps, s_z[wave][s][lane], hv, dl);
+        float pv[4], jv[4];
+        cell_jvp_z(prev, x, r, eps, s_z[wave][s][lane], dl, pv, jv);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+          dl[j] = jv[j] + (pv[j] - hv[j]);
           hl[j] = hv[j] + omega * dl[j];
           prev[j] = hv[j];
         }

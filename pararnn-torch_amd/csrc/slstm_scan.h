@@ -313,43 +313,17 @@ __device__ __forceinline__ void windowed_lookback(const TileId& id, int B, int n
   }
 }
 
-// The two gate exponents of a step: with the stabiliser m' = max(left, z_i) one
-// of f = e^(left - m') and i = e^(z_i - m') is exactly 1, the other e; al =
-// d m'/d left, ties split 0.5 / 0.5 (para_slstm.py:530-534), comes from the
-// difference in one clamped FMA (|left - z_i| > 1.5e-39 saturates it) instead of two
-// compares and two selects.
-struct Gates {
-  float f, i, al;
-};
-__device__ __forceinline__ Gates gate_split(float left, float zi) {
-  const float df = left - zi;
-  const float e = fexp(-fabsf(df));
-  const bool lf = df >= 0.f;
-  return Gates{lf ? 1.f : e, lf ? e : 1.f,
-               __builtin_amdgcn_fmed3f(fmaf(df, 3.4028235e38f, 0.5f), 0.f, 1.f)};
-}
-
 // Cell value and the per-channel Jacobian [out, in] over slots (c, n, m, h):
 //   c: [f, 0, cm, ch]   n: [0, f, nm, nh]   m: [0, 0, al, mh]
-//   h: inv * ((c row) - u * (n row)) + [0, 0, 0, g]
+//   h: inv * (c row) + dn * (n row) + [0, 0, 0, g]
 // The h row is kept factorised: h' = o c' / (n' + eps), so its derivative is
-// inv = o / den times that of c' less u = c' / den times that of n', plus g = u
-// do/dh through the output gate.  Applied to a vector that costs 3 operations for
-// the h row instead of 4, and the four dense h entries are never formed.
-// With dr = r_f - r_i and the gate split a1 = f (1 - al), a2 = i al, the m- and
-// h-derivatives of the c and n rows share their factors: cm = a1 c - a2 z, nm =
-// a1 n - a2, ch = dr cm + i (1 - z^2) r_z, nh = dr nm, and mh = r_i + al dr.  (dn =
-// -inv u is the n row's factor by itself, for the adjoint.)
-//
-// The Newton kernels are bound by vector issue (88-90% of the cycles), so what
-// counts is instructions: gate_split, differences like o - o^2 as one FMA, and sums
-// that start from the residual took pass 1 from 115 to 108 per step and pass 2 from
-// 68 to 62; B = 64, T = 2048, d = 1024, bf16, K = 3: 2.38 -> 2.27 ms.  (Applying dr
-// per vector here as well gives 2.25 ms, but lost accuracy where the iteration
-// diverges.)
+// inv = o / den times that of c', plus dn = -o c' / den^2 times that of n',
+// plus g = (c' / den) do/dh through the output gate.  Applied to a vector
+// that costs 3 operations for the h row instead of 4, and the four dense h
+// entries are never formed.
 struct CellJ {
   float pc, pn, pm, ph;
-  float f, cm, nm, al, inv, u, g, ch, nh, mh, dn;
+  float f, cm, ch, nm, nh, al, mh, inv, dn, g;
 };
 
 // The cell's z = tanh(z_z) at this step (it depends only on x and h).
@@ -367,33 +341,41 @@ __device__ __forceinline__ CellJ cell_jac_impl(const float prev[4], const float 
   const float zz = x[2] + r[2] * h;
   const float zo = x[3] + r[3] * h;
   const float left = zf + m;
-  const Gates gt = gate_split(left, zi);
-  const float f = gt.f, i = gt.i, al = gt.al;
+  const float mn = fmaxf(left, zi);
+  // d max(left, z_i) / d left, ties split 0.5 / 0.5 (para_slstm.py:530-534).
+  const float al = left > zi ? 1.f : (left == zi ? 0.5f : 0.f);
+  const float e = fexp(-fabsf(left - zi));  // the smaller of the two gate exponents
+  const bool lf = left >= zi;
+  const float f = lf ? 1.f : e;
+  const float i = lf ? e : 1.f;
   const float z = GIVEN_Z ? zg : ftanh5(zz);
   const float nn = f * n + i;
   const float cn = f * c + i * z;
   const float o = fsigmoid(zo);
   const float inv_den = frcp(nn + eps);
   CellJ J;
-  J.u = cn * inv_den;
   J.pc = cn;
   J.pn = nn;
-  J.pm = fmaxf(left, zi);
-  J.ph = o * J.u;
-  const float a1 = f - f * al;
+  J.pm = mn;
+  J.ph = o * (cn * inv_den);
+  // With d = r_f - r_i and the gate split a1 = f (1 - al), a2 = i al (al =
+  // d m'/d left), the m- and h-derivatives of the c and n rows share their
+  // factors: cm = a1 c - a2 z, nm = a1 n - a2, ch = d cm + i (1 - z^2) r_z,
+  // nh = d nm, and mh = r_i + al d.
+  const float a1 = f * (1.f - al);
   const float a2 = i * al;
+  const float dr = r[1] - r[0];
+  const float do_dh = o * (1.f - o) * r[3];
   J.f = f;
   J.al = al;
   J.cm = a1 * c - a2 * z;
   J.nm = a1 * n - a2;
-  J.inv = o * inv_den;
-  const float or3 = o * r[3];
-  J.g = J.u * (or3 - o * or3);
-  const float dr = r[1] - r[0];
   J.ch = dr * J.cm + i * ((1.f - z * z) * r[2]);
   J.nh = dr * J.nm;
   J.mh = r[0] + al * dr;
-  J.dn = -J.inv * J.u;
+  J.inv = o * inv_den;
+  J.dn = -J.inv * (cn * inv_den);
+  J.g = (cn * inv_den) * do_dh;
   return J;
 }
 
@@ -406,59 +388,80 @@ __device__ __forceinline__ CellJ cell_jac_z(const float prev[4], const float x[4
   return cell_jac_impl<true>(prev, x, r, eps, z);
 }
 
-// v <- J v + f(prev, x) - hv, without forming J (a forward-mode pass through the
-// cell, about half the arithmetic of building its entries and multiplying): the
-// step of the Newton scan from a known delta v.  z = cell_z(prev, x, r) given
-// (GIVEN_Z) or evaluated here.
+// Cell value p = f(prev, x) and the directional derivative jv = J v along
+// v, without forming J (a forward-mode pass through the cell, about half the
+// arithmetic of building the 12 entries and multiplying).
+// cell_jvp with z = cell_z(prev, x, r) given (GIVEN_Z) or evaluated here.
 template <bool GIVEN_Z>
-__device__ __forceinline__ void cell_delta(const float prev[4], const float x[4],
-                                           const float r[4], float eps, float zg,
-                                           const float hv[4], float v[4]) {
+__device__ __forceinline__ void cell_jvp_impl(const float prev[4], const float x[4],
+                                              const float r[4], float eps, float zg,
+                                              const float v[4], float p[4], float jv[4]) {
   const float c = prev[0], n = prev[1], m = prev[2], h = prev[3];
   const float zi = x[0] + r[0] * h;
   const float zf = x[1] + r[1] * h;
   const float zz = x[2] + r[2] * h;
   const float zo = x[3] + r[3] * h;
   const float left = zf + m;
-  const Gates gt = gate_split(left, zi);
-  const float f = gt.f, i = gt.i, al = gt.al;
+  const float mn = fmaxf(left, zi);
+  const float al = left > zi ? 1.f : (left == zi ? 0.5f : 0.f);
+  const float e = fexp(-fabsf(left - zi));
+  const bool lf = left >= zi;
+  const float f = lf ? 1.f : e;
+  const float i = lf ? e : 1.f;
   const float z = GIVEN_Z ? zg : ftanh5(zz);
   const float nn = f * n + i;
   const float cn = f * c + i * z;
   const float o = fsigmoid(zo);
   const float inv_den = frcp(nn + eps);
   const float u = cn * inv_den;
+  p[0] = cn;
+  p[1] = nn;
+  p[2] = mn;
+  p[3] = o * u;
+  // tangents: z_g' = r_g h', left' = z_f' + m', m_new' = al left' + (1 - al) z_i';
+  // with q = left' - z_i' = m' + (r_f - r_i) h', the gate tangents are
+  // f' = f (1 - al) q and i' = -i al q.
   const float q = v[2] + (r[1] - r[0]) * v[3];
-  const float a1 = f - f * al;
+  const float dmn = r[0] * v[3] + al * q;
+  const float a1 = f * (1.f - al);
   const float a2 = i * al;
   const float dnn = f * v[1] + q * (a1 * n - a2);
   const float dcn = f * v[0] + q * (a1 * c - a2 * z) + i * (1.f - z * z) * (r[2] * v[3]);
-  const float oh = o * (r[3] * v[3]);
-  const float dso = oh - o * oh;
-  v[0] = dcn + (cn - hv[0]);
-  v[1] = dnn + (nn - hv[1]);
-  v[2] = al * q + (r[0] * v[3] + (fmaxf(left, zi) - hv[2]));
-  v[3] = o * inv_den * (dcn - u * dnn) + (dso * u + (o * u - hv[3]));
+  const float dso = o * (1.f - o) * (r[3] * v[3]);
+  jv[0] = dcn;
+  jv[1] = dnn;
+  jv[2] = dmn;
+  jv[3] = dso * u + o * inv_den * (dcn - u * dnn);
+}
+
+__device__ __forceinline__ void cell_jvp(const float prev[4], const float x[4], const float r[4],
+                                         float eps, const float v[4], float p[4], float jv[4]) {
+  cell_jvp_impl<false>(prev, x, r, eps, 0.f, v, p, jv);
+}
+__device__ __forceinline__ void cell_jvp_z(const float prev[4], const float x[4],
+                                           const float r[4], float eps, float z, const float v[4],
+                                           float p[4], float jv[4]) {
+  cell_jvp_impl<true>(prev, x, r, eps, z, v, p, jv);
 }
 
 // v <- J v
 __device__ __forceinline__ void jmv(const CellJ& J, float v[4]) {
-  const float m = v[2], h = v[3];
-  v[0] = J.f * v[0] + J.cm * m + J.ch * h;
-  v[1] = J.f * v[1] + J.nm * m + J.nh * h;
+  const float c = v[0], n = v[1], m = v[2], h = v[3];
+  v[0] = J.f * c + J.cm * m + J.ch * h;
+  v[1] = J.f * n + J.nm * m + J.nh * h;
   v[2] = J.al * m + J.mh * h;
-  v[3] = J.inv * (v[0] - J.u * v[1]) + J.g * h;
+  v[3] = J.inv * v[0] + J.dn * v[1] + J.g * h;
 }
 
 // v <- J v + F: the affine step of the Newton scan.
 __device__ __forceinline__ void jmv_affine(const CellJ& J, const float F[4], float v[4]) {
-  const float m = v[2], h = v[3];
-  const float tc = J.f * v[0] + J.cm * m + J.ch * h;
-  const float tn = J.f * v[1] + J.nm * m + J.nh * h;
+  const float c = v[0], n = v[1], m = v[2], h = v[3];
+  const float tc = J.f * c + J.cm * m + J.ch * h;
+  const float tn = J.f * n + J.nm * m + J.nh * h;
   v[0] = tc + F[0];
   v[1] = tn + F[1];
-  v[2] = J.al * m + (J.mh * h + F[2]);
-  v[3] = J.inv * (tc - J.u * tn) + (J.g * h + F[3]);
+  v[2] = J.al * m + J.mh * h + F[2];
+  v[3] = J.inv * tc + J.dn * tn + J.g * h + F[3];
 }
 
 // ---- eager-rounding cell (scan_backend='eager' with 16-bit storage) -------
