@@ -38,15 +38,15 @@ from torch import Tensor
 
 
 # The last offsets that passed the checks: weak references to the tensor given
-# and to the int64 one returned, each with its version counter (bumped by every
-# in-place write), so the solve and the ops it calls check one stream once,
+# and to the int64 ones returned for it, each with its version counter (bumped by
+# every in-place write), so the solve and the ops it calls check one stream once,
 # with one device-to-host copy.  With them the longest sequence's length, which
 # only decides how a stream is run (the kernels read the offsets themselves).
-_checked: tuple[tuple[tuple[weakref.ref, int], ...], int, int] | None = None
+_Checked = tuple[tuple[tuple[weakref.ref, int], ...], int, int]
+_checked: _Checked | None = None
 
 
-def _known(t: Tensor, time: int) -> bool:
-    c = _checked
+def _known(c: _Checked | None, t: Tensor, time: int) -> bool:
     return c is not None and c[1] == time and any(r() is t and v == t._version for r, v in c[0])
 
 
@@ -64,7 +64,12 @@ def validate_cu_seqlens(cu_seqlens: Tensor, time: int,
     if cu_seqlens.dim() != 1 or cu_seqlens.numel() < 2:
         raise ValueError(f"cu_seqlens must be (S+1,), got {tuple(cu_seqlens.shape)}")
     cs = cu_seqlens.to(dtype=torch.long, device=device or cu_seqlens.device)
-    if _known(cu_seqlens, time) or _known(cs, time):
+    c = _checked
+    if _known(c, cu_seqlens, time) or _known(c, cs, time):
+        if not _known(c, cs, time):
+            # another copy of known offsets (int32, or of another device): as known
+            refs = tuple((r, v) for r, v in c[0] if r() is not None)
+            _checked = (refs + ((weakref.ref(cs), cs._version),), c[1], c[2])
         return cs
     host = cs.cpu()
     if int(host[0]) != 0:
@@ -83,7 +88,7 @@ def longest_sequence(cs: Tensor, time: int) -> int:
     """Length of the longest sequence of checked offsets (no copy from the
     device when they are the last ones checked)."""
     c = _checked
-    if c is not None and _known(cs, time):
+    if _known(c, cs, time):
         return c[2]
     return int((cs[1:] - cs[:-1]).max())
 

@@ -196,6 +196,47 @@ def test_graph_replays(monkeypatch):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("walk", ["0", "1", None])
+def test_packed_call_with_int32_offsets_is_captured(walk, monkeypatch):
+    """Known int32 offsets: a repeated packed call reads nothing back, so it can be
+    captured; each replay equals the eager result."""
+    from pararnn_amd import ops
+
+    if walk is None:
+        monkeypatch.delenv("PARARNN_AMD_GRU_WALK", raising=False)
+    else:
+        monkeypatch.setenv("PARARNN_AMD_GRU_WALK", walk)
+    print(f"case packed int32 capture walk={walk}", flush=True)
+    p = _params(2, 64, 3)
+    mats = _mats(p)
+    g = torch.Generator().manual_seed(5)
+    cs = torch.tensor([0, 17, 33, 34, 90], dtype=torch.int32, device=DEV)
+    xs = [p.wx(torch.randn(1, 90, 8, generator=g)).to(DEV) for _ in range(3)]
+    wx = xs[0].clone()
+    h0 = (torch.rand(4, 128, generator=g) - 0.5).to(DEV)
+    gr = torch.randn(1, 90, 128, generator=g).to(DEV)
+
+    def call(w):
+        out = ops.newton_gru_head_fused(w, *mats, h0, cs, max_iters=3, omega=1.0)
+        return [out, *ops.gru_head_backward_fused(w, *mats, h0, out, gr, cs)]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(wx)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = call(wx)
+    for x in xs:
+        want = call(x)
+        wx.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(held, want):
+            assert torch.equal(a, b)
+
+
 def test_two_streams(monkeypatch):
     """Solves of two streams at once keep apart (a workspace each)."""
     from pararnn_amd import ops

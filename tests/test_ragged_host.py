@@ -131,3 +131,22 @@ def test_validated_offsets_are_checked_again_after_a_write():
     validate_cu_seqlens(cs, 7)
     with pytest.raises(ValueError, match="must equal time"):
         validate_cu_seqlens(cs, 8)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_known_offsets_are_not_read_again(dtype, monkeypatch):
+    """From the second call on nothing is read back, neither by the check nor for the
+    longest sequence of what it returned (under graph capture a read is an error):
+    also for int32 offsets, whose int64 form is made anew by each call."""
+    from pararnn_amd.ragged import longest_sequence
+
+    cs = torch.tensor([0, 3, 10, 12], dtype=dtype)
+    validate_cu_seqlens(cs, 12)
+
+    def read(*a, **k):
+        raise AssertionError("device read")
+
+    for name in ("cpu", "item", "tolist", "__int__", "__bool__", "__index__"):
+        monkeypatch.setattr(torch.Tensor, name, read)
+    for _ in range(3):
+        assert longest_sequence(validate_cu_seqlens(cs, 12), 12) == 7
