@@ -1428,9 +1428,11 @@ constexpr Shape kNewtonFusedF32{16, 4};
 // rectangular tile lengths (their packed bodies are one guarded, head-checked
 // loop: no spills); the single-iteration launches run shorter tiles.
 constexpr Shape kPicardPacked{24, 4};
-// no spills at 28 steps; N=16019, d=860, 95 sequences: 0.36 ms against 0.375 (32
-// steps, 7 registers spilled) and 0.75 ms as one launch per pass
-constexpr Shape kPicardPackedF32{28, 4};
+// the rectangular launch's tile: a stream and the same sequences as padded rows
+// then compose their carries alike.  With 28 steps (no spills, against 7 registers
+// here: N=16019, d=860, 95 sequences 0.36 against 0.375 ms, one launch per pass
+// 0.75) the gradients of the two differed by twice as much.
+constexpr Shape kPicardPackedF32 = kPicardF32;
 inline Shape picard_packed_shape(bool narrow) { return narrow ? kPicardPacked : kPicardPackedF32; }
 constexpr Shape kNewtonFusedPacked{20, 4};
 constexpr Shape kNewtonFusedPackedF32{12, 4};

@@ -1,6 +1,6 @@
 """float32 warm start (zero-hidden pass and all Picard passes in one launch) at
-the edges of its tiles (32 steps per wave, 128 per tile; packed streams 28 and
-112) against the frozen-gate recurrence walked in float64.
+the edges of its tiles (32 steps per wave, 128 per tile) against the frozen-gate
+recurrence walked in float64.
 
 Bar: m is a sum of at most T float32 terms and n, c, h follow it through e^{z - m},
 so a slot is off by at most about T u max(1, |m|) relative to its largest value
@@ -63,7 +63,8 @@ def test_rectangular(B, T, d, P, with_h0):
     _check(got, want, T, P)
 
 
-@pytest.mark.parametrize("lengths", [[1], [27, 1, 1], [28, 29], [111, 1, 130], [5] * 40])
+@pytest.mark.parametrize("lengths", [[1], [27, 1, 1], [28, 29], [111, 1, 130], [5] * 40,
+                                     [31, 1, 1], [32, 33], [127, 1, 130]])
 @pytest.mark.parametrize("P", [0, 3])
 def test_packed(lengths, P):
     d, N = 70, sum(lengths)
