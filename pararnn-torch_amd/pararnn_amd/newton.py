@@ -211,20 +211,27 @@ def _prepend_any(states: Tensor, h0: Tensor | None, cu_seqlens: Tensor | None) -
     return prepend_state_ragged(states, h0, cu_seqlens)
 
 
-def _max_residual(cell, wx, states, h0, cu_seqlens) -> float:
+def _max_residual(cell, wx, states, h0, cu_seqlens, x=None) -> float:
     """max |f(H_{t-1}, x_t) - H_t| on the host: one kernel over ``wx = W_x(x)`` and
-    the states.  A cell whose step is not the library's own is evaluated by that."""
+    the states.  A cell whose step is not the library's own is evaluated by that:
+    from ``x`` where the caller has it (a step of its own need not know ``wx``)."""
     def own(base: type, *names: str) -> bool:
         return isinstance(cell, base) and all(
             getattr(getattr(cell, n), "__func__", None) is getattr(base, n) for n in names)
 
-    if own(ParaSLSTM, "step", "_acts", "_recurrent"):
-        return float(ops.slstm_residual(wx, cell.clipped_r(), h0, states, cu_seqlens,
-                                        eps=cell.eps))
-    if own(ParaGRU, "step", "_acts") and cell.mix == "head":
-        return float(ops.gru_head_residual(wx, *cell.clipped_a_head(), h0, states, cu_seqlens))
-    pred = cell.step(_prepend_any(states, h0, cu_seqlens), None, wx=wx)
-    return float((pred - states).abs().amax())
+    slstm = own(ParaSLSTM, "step", "_acts", "_recurrent")
+    if slstm or (own(ParaGRU, "step", "_acts") and cell.mix == "head"):
+        with torch.no_grad():
+            if wx is None:
+                wx = cell.W_x(x)
+            if slstm:
+                return float(ops.slstm_residual(wx, cell.clipped_r(), h0, states, cu_seqlens,
+                                                eps=cell.eps))
+            return float(ops.gru_head_residual(wx, *cell.clipped_a_head(), h0, states,
+                                               cu_seqlens))
+    prev = _prepend_any(states, h0, cu_seqlens)
+    pred = cell.step(prev, None, wx=wx) if x is None else cell.step(prev, x)
+    return float((pred - states).detach().abs().amax())
 
 
 def _fill_stats(cell, x, states, h0, config, *, iters, stats, history=(), known=None,
@@ -234,9 +241,7 @@ def _fill_stats(cell, x, states, h0, config, *, iters, stats, history=(), known=
     if stats is None and config.residual_fail is None:
         return
     if known is None:
-        with torch.no_grad():
-            res = _max_residual(cell, cell.W_x(x) if wx is None else wx, states.detach(), h0,
-                                cu_seqlens)
+        res = _max_residual(cell, wx, states, h0, cu_seqlens, x=x)
     else:
         res = known
     hist = tuple(history)

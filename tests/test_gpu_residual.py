@@ -100,6 +100,23 @@ def test_own_step_of_a_subclass_is_evaluated():
     assert abs(st.max_residual - 1.0) < 1e-3
 
 
+@pytest.mark.parametrize("config", [{}, {"scan_backend": "eager", "residual_atol": None},
+                                    {"chunk_len": 8, "picard_adapt": False}])
+def test_step_without_wx_passes_the_default_gate(config):
+    """A step of two arguments that agrees with the library's: the gate accepts the solve."""
+    class Two(ParaSLSTM):
+        def step(self, state_prev, x):
+            return super().step(state_prev, x)
+
+    torch.manual_seed(0)
+    cell = Two(8, 16, device=DEV)
+    x = torch.randn(2, 20, 8, device=DEV) * 0.5
+    st = NewtonStats()
+    with torch.no_grad():
+        newton_apply(cell, x, NewtonConfig(**config), stats=st)
+    assert st.max_residual < 1e-3
+
+
 def test_residual_rejects_mismatched_operands():
     wx = torch.zeros(1, 4, 12, device=DEV)
     a = torch.zeros(1, 4, 4, device=DEV)
