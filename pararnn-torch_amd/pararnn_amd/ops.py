@@ -57,7 +57,7 @@ def _workspace(nbytes: int, dev: torch.device) -> Tensor:
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=dev)
 
 
-# Tagged sLSTM workspaces: one zero-filled buffer per (device, stream), kept
+# Tagged workspaces (sLSTM, head-GRU walks): one zero-filled buffer per (device, stream), kept
 # across calls, with a growing tag base, so a call skips clearing its
 # look-back words (prnn_slstm_*_ex).  Only the library writes these buffers;
 # calls on one stream run in order.  Graph capture takes a fresh, cleared
@@ -74,7 +74,7 @@ def _tagged_enabled() -> bool:
 
 
 def _slstm_workspace(nbytes: int, dev: torch.device) -> tuple[Tensor, int]:
-    """``(workspace, tag_base)`` for an sLSTM call on the current stream."""
+    """``(workspace, tag_base)`` for a tagged call on the current stream."""
     if not _tagged_enabled() or torch.cuda.is_current_stream_capturing():
         return _workspace(nbytes, dev), 0
     stream = torch.cuda.current_stream(dev)
@@ -82,7 +82,10 @@ def _slstm_workspace(nbytes: int, dev: torch.device) -> tuple[Tensor, int]:
     with _tagged_lock:
         ent = _tagged.get(key)
         if ent is None or ent[0].numel() < nbytes or ent[1] + _TAG_SPAN > _TAG_BASE_MAX:
-            # Zero-filled on this stream, ahead of the call that uses it.
+            # Zero-filled on this stream, ahead of the call that uses it; the
+            # buffer that it replaces is given back first.
+            ent = None
+            _tagged.pop(key, None)
             ent = [torch.zeros(max(int(nbytes), 256), dtype=torch.uint8, device=dev), 1]
             _tagged[key] = ent
         _tagged.move_to_end(key)
@@ -111,7 +114,7 @@ def _check_lookback(ws: Tensor, what: str) -> None:
 
 
 def release_workspaces() -> None:
-    """Drop the cached sLSTM workspaces (they are re-created on demand)."""
+    """Drop the cached tagged workspaces (they are re-created on demand)."""
     with _tagged_lock:
         _tagged.clear()
 
@@ -682,6 +685,23 @@ def _walks(units: int, total: int, longest: int, iters: int) -> bool:
     return 1.15 * walk < chunk
 
 
+def _walk_workspace(nbytes: int, dev: torch.device) -> tuple[Tensor, int] | None:
+    """``(workspace, tag_base)`` of a walk solve, 8 (K - 1) bytes per element: kept for
+    the stream up to ``_WALK_KEEP`` bytes, beyond that of this call alone and cleared by
+    it (the clear is a few per cent of a solve of that size).  None where it would take
+    more than ``_wide_workspace_cap`` or than there is: the chunked scan's
+    workspace does not grow with K (at K = 3 it is the larger one)."""
+    if nbytes > _wide_workspace_cap(dev):
+        return None
+    try:
+        if nbytes <= _WALK_KEEP:
+            return _slstm_workspace(nbytes, dev)
+        return _workspace(nbytes, dev), 0
+    except torch.OutOfMemoryError:
+        return None
+
+
+_WALK_KEEP = 512 << 20
 _WALK_MAX_ITERS = 64  # PRNN_TAG_SPAN
 _CHUNK_SWITCHES = ("PRNN_GRU_REPLAY_MFMA", "PRNN_GRU_REV_MFMA", "PRNN_GRU_CARRY_SINGLE")
 
@@ -712,17 +732,20 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
                                  time if cs is None else longest_sequence(cs, time), max_iters):
         nbytes = lib.prnn_gru_head_walk_newton_workspace_size(batch, time, hb.n_blocks,
                                                               int(max_iters))
-    if 0 < nbytes <= _wide_workspace_cap(wx.device):
+    if nbytes > 0:
         with torch.cuda.device(wx.device):
-            ws, tag = _slstm_workspace(nbytes, wx.device)
-            rc = lib.prnn_gru_head_walk_newton(
-                _ptr(wx), _ptr(a_z), _ptr(a_r), _ptr(a_n), _ptr(h0), _ptr(out), batch, time,
-                hb.n_blocks, int(max_iters), float(omega), code, _ptr(cs32),
-                0 if cs is None else rows, _ptr(ws), ws.numel(), tag, _stream(wx.device),
-            )
-        _lib.check(rc, "newton_gru_head_fused")
-        _check_lookback(ws, "newton_gru_head_fused")
-        return _from_blocks(hb, [(out, 1)])[0][0]
+            held = _walk_workspace(nbytes, wx.device)
+            if held is not None:
+                ws, tag = held
+                rc = lib.prnn_gru_head_walk_newton(
+                    _ptr(wx), _ptr(a_z), _ptr(a_r), _ptr(a_n), _ptr(h0), _ptr(out), batch, time,
+                    hb.n_blocks, int(max_iters), float(omega), code, _ptr(cs32),
+                    0 if cs is None else rows, _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                )
+        if held is not None:
+            _lib.check(rc, "newton_gru_head_fused")
+            _check_lookback(ws, "newton_gru_head_fused")
+            return _from_blocks(hb, [(out, 1)])[0][0]
     with torch.cuda.device(wx.device):
         if cs is None:
             nbytes = lib.prnn_gru_head_newton_workspace_size(batch, time, hb.n_blocks, 64,

@@ -259,3 +259,31 @@ def test_two_streams(monkeypatch):
     for i in range(2):
         for o in got[i]:
             assert torch.equal(o, want[i])
+
+
+@pytest.mark.parametrize("room", ["kept", "own", "none"])
+def test_each_workspace_gives_the_same_states(room, monkeypatch):
+    """From the stream's cache, from a buffer of the call's own (other values in it), and
+    with no room for either (the chunked scan, at its own bar); nothing of a buffer of
+    the call's own stays."""
+    from pararnn_amd import ops
+
+    monkeypatch.setenv("PARARNN_AMD_GRU_WALK", "1")
+    monkeypatch.setenv("PARARNN_AMD_CHECK_STATUS", "1")
+    print(f"case workspace {room}", flush=True)
+    p = _params(3, 64, 9)
+    wx = p.wx(torch.randn(4, 300, 8, generator=torch.Generator().manual_seed(9))).to(DEV)
+    want = ops.newton_gru_head_fused(wx, *_mats(p), max_iters=3, omega=1.0)
+    ops.release_workspaces()
+    if room != "kept":
+        monkeypatch.setattr(ops, "_WALK_KEEP", 0)
+    if room == "none":
+        monkeypatch.setattr(ops, "_wide_workspace_cap", lambda d: 0)
+    torch.full((1 << 24,), float("nan"), device=DEV)  # what a fresh buffer may hold
+    for _ in range(2):
+        got = ops.newton_gru_head_fused(wx, *_mats(p), max_iters=3, omega=1.0)
+        if room == "none":
+            assert (got - want).abs().max().item() <= 1e-5
+        else:
+            assert torch.equal(got, want)
+    assert bool(ops._tagged) is (room == "kept")

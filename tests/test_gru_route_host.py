@@ -48,3 +48,59 @@ def test_longest_sequence_follows_the_offsets():
     assert longest_sequence(validate_cu_seqlens(cs, 12), 12) == 9
     other = torch.tensor([0, 5, 12])
     assert longest_sequence(other, 12) == 7
+
+
+def test_walk_workspaces_kept_are_bounded(monkeypatch):
+    """Small ones come from the stream's cache, larger ones belong to the call (tag 0: it
+    clears them), and what is over the cap or not to be had sends the call to the scan."""
+    import torch
+
+    dev = torch.device("cuda", 0)
+    full = []
+
+    def temporary(n, d):
+        if full:
+            raise torch.OutOfMemoryError("no room")
+        return "own"
+
+    monkeypatch.setattr(ops, "_wide_workspace_cap", lambda d: 1 << 33)
+    monkeypatch.setattr(ops, "_workspace", temporary)
+    monkeypatch.setattr(ops, "_slstm_workspace", lambda n, d: (temporary(n, d) and "kept", 65))
+    keep = ops._WALK_KEEP
+    assert keep <= 1 << 30
+    assert ops._walk_workspace(keep, dev) == ("kept", 65)
+    assert ops._walk_workspace(keep + 1, dev) == ("own", 0)
+    assert ops._walk_workspace((1 << 33) + 1, dev) is None
+    full.append(1)
+    assert ops._walk_workspace(keep, dev) is None and ops._walk_workspace(keep + 1, dev) is None
+
+
+def test_a_growing_cache_gives_its_buffer_back_first(monkeypatch):
+    import gc
+    import weakref
+
+    import torch
+
+    class _S:
+        cuda_stream = 77
+
+    alive = []
+    real = torch.zeros
+
+    def zeros(n, dtype, device):
+        gc.collect()
+        alive.append([r() is not None for r in made])
+        out = real(n, dtype=dtype)
+        made.append(weakref.ref(out))
+        return out
+
+    made = []
+    monkeypatch.setattr(ops.torch, "zeros", zeros)
+    monkeypatch.setattr(ops.torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops.torch.cuda, "current_stream", lambda d: _S)
+    ops.release_workspaces()
+    dev = torch.device("cuda", 0)
+    for n in (1024, 4096, 65536):
+        ops._slstm_workspace(n, dev)
+    assert alive == [[], [False], [False, False]]
+    ops.release_workspaces()
