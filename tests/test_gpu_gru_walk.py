@@ -287,3 +287,32 @@ def test_each_workspace_gives_the_same_states(room, monkeypatch):
         else:
             assert torch.equal(got, want)
     assert bool(ops._tagged) is (room == "kept")
+
+
+def test_threads_on_one_stream(monkeypatch):
+    """Four threads on the default stream, each with solves of its own."""
+    import threading
+
+    from pararnn_amd import ops
+
+    monkeypatch.setenv("PARARNN_AMD_GRU_WALK", "1")
+    print("case four threads, one stream", flush=True)
+    p = _params(2, 64, 6)
+    mats = _mats(p)
+    g = torch.Generator().manual_seed(8)
+    xs = [p.wx(torch.randn(2 + i, 200, 8, generator=g)).to(DEV) for i in range(4)]
+    want = [ops.newton_gru_head_fused(x, *mats, max_iters=3, omega=1.0) for x in xs]
+    got = [[] for _ in xs]
+
+    def work(i):
+        for _ in range(10):
+            got[i].append(ops.newton_gru_head_fused(xs[i], *mats, max_iters=3, omega=1.0))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for w, outs in zip(want, got):
+        assert len(outs) == 10 and all(torch.equal(o, w) for o in outs)

@@ -104,3 +104,59 @@ def test_a_growing_cache_gives_its_buffer_back_first(monkeypatch):
         ops._slstm_workspace(n, dev)
     assert alive == [[], [False], [False, False]]
     ops.release_workspaces()
+
+
+def test_threads_on_one_stream_take_turns(monkeypatch):
+    """From picking the tag to the launch (buffers on the CPU, a library that only looks):
+    two calls at once would clear one buffer's tickets twice and then launch twice."""
+    import contextlib
+    import threading
+    import time
+
+    import torch
+
+    inside, seen, wrong = [], [], []
+
+    class _Lib:
+        def prnn_gru_head_walk_newton_workspace_size(self, *a):
+            return 4096
+
+        def prnn_gru_head_walk_newton(self, *a):
+            tag = a[-2]
+            if inside:
+                wrong.append(("together", tag))
+            inside.append(tag)
+            time.sleep(0.02)
+            seen.append(tag)
+            inside.pop()
+            return 0
+
+    class _S:
+        cuda_stream = 0
+
+    monkeypatch.setattr(ops._lib, "load", _Lib)
+    monkeypatch.setattr(ops._lib, "check", lambda rc, what: None)
+    monkeypatch.setattr(ops, "_validate", lambda *a: 0)
+    monkeypatch.setattr(ops, "_stream", lambda d: 0)
+    monkeypatch.setattr(ops, "_walks", lambda *a: True)
+    monkeypatch.setattr(ops, "_wide_workspace_cap", lambda d: 1 << 30)
+    monkeypatch.setattr(ops.torch.cuda, "device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(ops.torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(ops.torch.cuda, "current_stream", lambda d: _S)
+    monkeypatch.setattr(ops.torch.cuda, "is_current_stream_capturing", lambda: False)
+    ops.release_workspaces()
+    a = torch.zeros(1, 64, 64)
+    wx = torch.zeros(1, 3, 192)
+
+    def work():
+        for _ in range(5):
+            ops._gru_head_dense(wx, a, a, a, None, 3, 1.0)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    ops.release_workspaces()
+    assert not wrong and len(seen) == 20
+    assert seen == sorted(set(seen))  # launched in the order of their tags
