@@ -63,7 +63,10 @@ def _workspace(nbytes: int, dev: torch.device) -> Tensor:
 # calls on one stream run in order.  Graph capture takes a fresh, cleared
 # workspace per call (a replay would repeat captured tags).
 _TAG_SPAN = 64           # PRNN_TAG_SPAN
-_TAG_BASE_MAX = 1 << 30  # PRNN_TAG_BASE_MAX
+# Largest tag base before a fresh buffer (PRNN_TAG_BASE_MAX allows 2^30).  Calls lay the
+# buffer out differently, and the sLSTM backward keeps float32 partial sums behind its
+# words, which a later call may read as words: below 2^23 no tag is a normal float's bits.
+_TAG_BASE_MAX = (1 << 23) - _TAG_SPAN
 _TAGGED_MAX = 4          # cached buffers (least recently used dropped first)
 _tagged_lock = threading.Lock()
 _tagged: collections.OrderedDict[tuple[int, int], list] = collections.OrderedDict()

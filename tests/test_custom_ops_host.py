@@ -110,3 +110,15 @@ def test_tagged_workspace_cache_is_bounded(monkeypatch):
     assert all(b == 1 for b in bases) and len(made) == 10
     ops.release_workspaces()
     assert not ops._tagged
+
+
+def test_no_tag_is_the_bit_pattern_of_a_normal_float():
+    """A kept buffer holds words of one call where another had float32 partial sums: a
+    tag (base .. base + 63, in the upper half of a word) must not be what a sum looks like."""
+    import numpy as np
+
+    from pararnn_amd import ops
+
+    top = np.array([ops._TAG_BASE_MAX], dtype=np.uint32).view(np.float32)[0]
+    assert 0 < top < np.finfo(np.float32).smallest_normal
+    assert ops._TAG_BASE_MAX >= 1000 * ops._TAG_SPAN  # re-zeroed once in many calls
