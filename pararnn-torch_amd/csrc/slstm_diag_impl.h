@@ -233,15 +233,13 @@ template <typename TX, int L, int W, bool DET>
 static void launch_frozen(bool has_h, bool full_out, const TX* wx, const TX* r, const TX* h0,
                           const TX* src, TX* out_full, TX* out_h, int B, int T, int d, float eps,
                           const Lookback& lb, int epoch, hipStream_t stream) {
-  constexpr bool PK = false;
-  const Packed pk{nullptr, nullptr, 0};
   const Geo g = geometry(B, T, d, Shape{L, W});
   const dim3 grid(g.n_tiles), block(64 * W);
   int* ctr = lb.counters + epoch;
 #define PRNN_FROZEN(HH, FO)                                                                    \
-  slstm_frozen_kernel<TX, L, W, HH, FO, DET, PK><<<grid, block, 0, stream>>>(                  \
+  slstm_frozen_kernel<TX, L, W, HH, FO, DET><<<grid, block, 0, stream>>>(                      \
       wx, r, h0, src, out_full, out_h, B, T, d, g.n_cb, eps, ctr, lb.agg, lb.incl,             \
-      lb.tag_base + epoch, lb.spin(), pk)
+      lb.tag_base + epoch, lb.spin())
   if (has_h) {
     if (full_out) PRNN_FROZEN(true, true); else PRNN_FROZEN(true, false);
   } else {

@@ -165,12 +165,12 @@ struct PreStash<float> {
 // lane owns one channel; its L steps are read once (pass 1, which builds the
 // lane aggregate), kept in registers through the look-back, and replayed from
 // the true carry in pass 2, which writes the trajectory.
-template <typename TX, int L, int W, bool HAS_H, bool FULL_OUT, bool DET, bool PK>
+template <typename TX, int L, int W, bool HAS_H, bool FULL_OUT, bool DET>
 __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
     const TX* __restrict__ wx, const TX* __restrict__ rmix, const TX* __restrict__ h0,
     const TX* __restrict__ hsrc, TX* __restrict__ out_full, TX* __restrict__ out_h, int B, int T,
     int d, int n_cb, float eps, int* __restrict__ counter, unsigned long long* __restrict__ agg,
-    unsigned long long* __restrict__ incl, int epoch, Spin spin, Packed pk) {
+    unsigned long long* __restrict__ incl, int epoch, Spin spin) {
   constexpr int KP = 2;  // predecessors per wave per look-back round
   using Stash = PreStash<TX>;
   constexpr uint32_t SZ = sizeof(TX);
@@ -204,12 +204,6 @@ __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
       hp0 = ld(h0 + static_cast<size_t>(id.b) * row4 + 3 * d + c0 + lane);
   }
 
-  // Packed sequences: heads among this wave's steps (see Packed); a head
-  // restarts the state from its sequence's initial one.
-  Heads hd{0ull, 0};
-  if constexpr (PK) hd = find_heads(pk, t0, n_steps);
-  auto head_of = [&](int s, float st[4]) { head_state(pk, h0, hd.seq(s), d, c0 + lane, live, st); };
-
   // Pass 1: read the steps, stash the pre-activations, and fold the segment
   // aggregate from the empty state (m = -inf, n = c = 0).
   uint32_t stash[L][Stash::N];
@@ -217,41 +211,29 @@ __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
   {
     const rsrc_t rx = make_rsrc(wx + first * row4 + c0, span4);
     const rsrc_t rh = make_rsrc(HAS_H ? hsrc + first * d + c0 : nullptr, HAS_H ? span1 : 0);
-    auto step = [&](int s, auto chk) {
-      constexpr bool CHECK = decltype(chk)::value;
-      const bool head = CHECK && hd.at(s);
-      float hs[4];
-      if (head) head_of(s, hs);
+    auto step = [&](int s) {
       uint32_t x[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         x[g] = ldb_bits(static_cast<TX*>(nullptr), rx, voff, s * row4 * SZ + g * slot);
       float hp = hp0;
       if (HAS_H && s > 0) hp = ldb<TX>(rh, voff, (s - 1) * d * SZ);
-      if (head) hp = hs[3];
       Stash::template make<HAS_H>(x, r, hp, stash[s]);
       float p[4];
       Stash::get(stash[s], p);
-      if (head) a = FG{-INFINITY, hs[2], hs[1], hs[0]};
       a.F += p[1];
       fg_step(p[0], p[1], p[2], a.M, a.N, a.C);
     };
     // Whole segments run branch-free so the loads of many steps are in
     // flight together; only the last segment of a sequence is guarded.
-    auto run = [&](auto chk) {
-      if (n_steps == L) {
+    if (n_steps == L) {
 #pragma unroll
-        for (int s = 0; s < L; ++s) step(s, chk);
-      } else {
+      for (int s = 0; s < L; ++s) step(s);
+    } else {
 #pragma unroll
-        for (int s = 0; s < L; ++s)
-          if (s < n_steps) step(s, chk);
-      }
-    };
-    if (PK && hd.mask)
-      run(std::true_type{});
-    else
-      run(std::false_type{});
+      for (int s = 0; s < L; ++s)
+        if (s < n_steps) step(s);
+    }
   }
   s_agg[wave][0][lane] = a.F;
   s_agg[wave][1][lane] = a.M;
@@ -267,7 +249,7 @@ __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
       tile_agg = fg_compose(
           tile_agg, FG{s_agg[w][0][lane], s_agg[w][1][lane], s_agg[w][2][lane], s_agg[w][3][lane]});
     if (id.chunk == 0) {
-      if (!PK && h0 != nullptr && live) {
+      if (h0 != nullptr && live) {
         const TX* hb = h0 + static_cast<size_t>(id.b) * row4 + c0 + lane;
         carry[2] = ld(hb);
         carry[1] = ld(hb + d);
@@ -314,15 +296,7 @@ __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
   float m = s_carry[wave][0][lane], n = s_carry[wave][1][lane], c = s_carry[wave][2][lane];
   const rsrc_t ro = FULL_OUT ? make_rsrc(out_full + first * row4 + c0, span4)
                              : make_rsrc(out_h + first * d + c0, span1);
-  auto replay = [&](int s, auto chk) {
-    constexpr bool CHECK = decltype(chk)::value;
-    if (CHECK && hd.at(s)) {
-      float hs[4];
-      head_of(s, hs);
-      c = hs[0];
-      n = hs[1];
-      m = hs[2];
-    }
+  auto replay = [&](int s) {
     float p[4];
     Stash::get(stash[s], p);
     fg_step(p[0], p[1], p[2], m, n, c);
@@ -338,20 +312,14 @@ __global__ __launch_bounds__(64 * W) void slstm_frozen_kernel(
       stb<TX>(ro, voff, s * d * SZ, h);
     }
   };
-  auto run2 = [&](auto chk) {
-    if (n_steps == L) {
+  if (n_steps == L) {
 #pragma unroll
-      for (int s = 0; s < L; ++s) replay(s, chk);
-    } else {
+    for (int s = 0; s < L; ++s) replay(s);
+  } else {
 #pragma unroll
-      for (int s = 0; s < L; ++s)
-        if (s < n_steps) replay(s, chk);
-    }
-  };
-  if (PK && hd.mask)
-    run2(std::true_type{});
-  else
-    run2(std::false_type{});
+    for (int s = 0; s < L; ++s)
+      if (s < n_steps) replay(s);
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -18,8 +18,9 @@ have zero inputs, zero weights and zero initial state, so they stay at zero
 (z = r = 1/2, n = 0 gives h' = h / 2) and never touch a real channel.
 
 The solves and their backward move everything a call needs in one launch
-(``ops._move_blocks``, ``csrc/gru_blocks.hip``); the tensor-op forms here serve the
-decode weights, which are laid out once, and the CPU.
+(``ops._move_blocks``, ``csrc/gru_blocks.hip``); of the tensor-op forms here
+``matrices`` serves the decode weights, which are laid out once, and the others are
+what the tests hold the moves against.
 
 The reference handles ``d_head <= 64`` with a masked ``BLOCK_D`` tile
 (kernels/newton_gru_head.py:121-136).  Heads of 64 < d_head <= 128 take the
