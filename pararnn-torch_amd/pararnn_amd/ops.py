@@ -82,20 +82,21 @@ def _stream_key(dev: torch.device) -> tuple[int, int]:
     return index, torch.cuda.current_stream(dev).cuda_stream
 
 
-def _one_at_a_time(dev: torch.device) -> threading.RLock:
-    """The lock of tagged calls on the current stream."""
-    return _stream_locks[hash(_stream_key(dev)) % len(_stream_locks)]
+def _one_at_a_time(key: tuple[int, int]) -> threading.RLock:
+    """The lock of tagged calls on a stream (``_stream_key``)."""
+    return _stream_locks[hash(key) % len(_stream_locks)]
 
 
 def _tagged_enabled() -> bool:
     return os.environ.get("PARARNN_AMD_TAGGED_WS", "1") != "0"
 
 
-def _slstm_workspace(nbytes: int, dev: torch.device) -> tuple[Tensor, int]:
-    """``(workspace, tag_base)`` for a tagged call on the current stream."""
+def _slstm_workspace(nbytes: int, dev: torch.device,
+                     key: tuple[int, int] | None = None) -> tuple[Tensor, int]:
+    """``(workspace, tag_base)`` for a tagged call on the current stream (of ``key``)."""
     if not _tagged_enabled() or torch.cuda.is_current_stream_capturing():
         return _workspace(nbytes, dev), 0
-    key = _stream_key(dev)
+    key = key or _stream_key(dev)
     with _tagged_lock:
         ent = _tagged.get(key)
         if ent is None or ent[0].numel() < nbytes or ent[1] + _TAG_SPAN > _TAG_BASE_MAX:
@@ -222,17 +223,18 @@ def slstm_init_fused(
     out = wx.new_empty(batch, time, 4, d_h)
     lib = _lib.load()
     _lib.sync_deterministic(lib)
-    with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
+    key = _stream_key(wx.device)
+    with torch.cuda.device(wx.device), _one_at_a_time(key):
         if cs32 is None:
             nbytes = lib.prnn_slstm_init_workspace_size(batch, time, d_h, picard_iters, code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_init_ex(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(out), batch, time, d_h, int(picard_iters),
                 float(eps), code, _ptr(ws), ws.numel(), tag, _stream(wx.device),
             )
         else:
             nbytes = lib.prnn_slstm_init_packed_workspace_size(time, d_h, picard_iters, code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_init_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(out), time, d_h, int(picard_iters),
                 float(eps), code, _ptr(cs32), n_seq, _ptr(bt), _ptr(ws), ws.numel(), tag,
@@ -310,10 +312,11 @@ def newton_slstm_fused(
     out = wx.new_empty(batch, time, 4, d_h)
     lib = _lib.load()
     _lib.sync_deterministic(lib)
-    with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
+    key = _stream_key(wx.device)
+    with torch.cuda.device(wx.device), _one_at_a_time(key):
         if cs32 is None:
             nbytes = lib.prnn_slstm_newton_workspace_size(batch, time, d_h, int(max_iters), code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_ex(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), batch, time, d_h,
                 int(max_iters), float(omega), float(eps), code, _ptr(ws), ws.numel(), tag,
@@ -321,7 +324,7 @@ def newton_slstm_fused(
             )
         else:
             nbytes = lib.prnn_slstm_newton_packed_workspace_size(time, d_h, int(max_iters), code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), time, d_h,
                 int(max_iters), float(omega), float(eps), code, _ptr(cs32), n_seq, _ptr(bt),
@@ -355,10 +358,11 @@ def slstm_newton_step(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor, 
     out = torch.empty(batch, time, 4, d_h, dtype=torch.float32, device=wx.device)
     lib = _lib.load()
     _lib.sync_deterministic(lib)
-    with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
+    key = _stream_key(wx.device)
+    with torch.cuda.device(wx.device), _one_at_a_time(key):
         if cs32 is None:
             nbytes = lib.prnn_slstm_newton_workspace_size(batch, time, d_h, 1, code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_step(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), int(in_f32), _ptr(out), batch, time,
                 d_h, float(omega), float(eps), code, _ptr(ws), ws.numel(), tag,
@@ -366,7 +370,7 @@ def slstm_newton_step(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor, 
             )
         else:
             nbytes = lib.prnn_slstm_newton_packed_workspace_size(time, d_h, 1, code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_step_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), int(in_f32), _ptr(out), time, d_h,
                 float(omega), float(eps), code, _ptr(cs32), n_seq, _ptr(bt), _ptr(ws),
@@ -397,17 +401,18 @@ def slstm_newton_eager(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor,
     out = torch.empty_like(states)
     lib = _lib.load()
     _lib.sync_deterministic(lib)
-    with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
+    key = _stream_key(wx.device)
+    with torch.cuda.device(wx.device), _one_at_a_time(key):
         if cs32 is None:
             nbytes = lib.prnn_slstm_newton_workspace_size(batch, time, d_h, 1, code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_eager(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), batch, time, d_h,
                 float(omega), float(eps), code, _ptr(ws), ws.numel(), tag, _stream(wx.device),
             )
         else:
             nbytes = lib.prnn_slstm_newton_packed_workspace_size(time, d_h, 1, code)
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_eager_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), time, d_h, float(omega),
                 float(eps), code, _ptr(cs32), n_seq, _ptr(bt), _ptr(ws), ws.numel(), tag,
@@ -460,9 +465,10 @@ def slstm_backward_fused(
     g_b = torch.empty(4, d_h, dtype=torch.float32, device=wx.device)
     lib = _lib.load()
     _lib.sync_deterministic(lib)
-    with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
+    key = _stream_key(wx.device)
+    with torch.cuda.device(wx.device), _one_at_a_time(key):
         nbytes = lib.prnn_slstm_backward_workspace_size(batch, time, d_h, code)
-        ws, tag = _slstm_workspace(nbytes, wx.device)
+        ws, tag = _slstm_workspace(nbytes, wx.device, key)
         if cs32 is None:
             rc = lib.prnn_slstm_backward_ex(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(grad), _ptr(g_wx), _ptr(g_r),
@@ -702,7 +708,8 @@ def _walks(units: int, total: int, longest: int, iters: int) -> bool:
     return 1.15 * walk < chunk
 
 
-def _walk_workspace(nbytes: int, dev: torch.device) -> tuple[Tensor, int] | None:
+def _walk_workspace(nbytes: int, dev: torch.device,
+                    key: tuple[int, int]) -> tuple[Tensor, int] | None:
     """``(workspace, tag_base)`` of a walk solve, 8 (K - 1) bytes per element: kept for
     the stream up to ``_WALK_KEEP`` bytes, beyond that of this call alone and cleared by
     it (8 heads, T = 2048, K = 3: 2.04 -> 2.12 ms at B = 33, 2.96 -> 3.13 at B = 64).  None where it would take
@@ -712,7 +719,7 @@ def _walk_workspace(nbytes: int, dev: torch.device) -> tuple[Tensor, int] | None
         return None
     try:
         if nbytes <= _WALK_KEEP:
-            return _slstm_workspace(nbytes, dev)
+            return _slstm_workspace(nbytes, dev, key)
         return _workspace(nbytes, dev), 0
     except torch.OutOfMemoryError:
         return None
@@ -750,8 +757,9 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
         nbytes = lib.prnn_gru_head_walk_newton_workspace_size(batch, time, hb.n_blocks,
                                                               int(max_iters))
     if nbytes > 0:
-        with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
-            held = _walk_workspace(nbytes, wx.device)
+        key = _stream_key(wx.device)
+        with torch.cuda.device(wx.device), _one_at_a_time(key):
+            held = _walk_workspace(nbytes, wx.device, key)
             if held is not None:
                 ws, tag = held
                 rc = lib.prnn_gru_head_walk_newton(
@@ -999,8 +1007,9 @@ def _gru_head_wide(wx, a_z, a_r, a_n, h0, max_iters, omega, code, cs=None):
         out = wx.new_empty(batch, time, d_h)
         h0_c = None if h0_32 is None else h0_32.contiguous()
         guess = states.contiguous()
-        with torch.cuda.device(wx.device), _one_at_a_time(wx.device):
-            ws, tag = _slstm_workspace(nbytes, wx.device)
+        key = _stream_key(wx.device)
+        with torch.cuda.device(wx.device), _one_at_a_time(key):
+            ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_gru_wide_newton(
                 _ptr(wx_c), _ptr(a_k[0]), _ptr(a_k[1]), _ptr(a_k[2]), _ptr(h0_c), _ptr(guess),
                 _ptr(out), batch, time, n_heads, d_head, max_iters, float(omega), code,

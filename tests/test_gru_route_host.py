@@ -65,14 +65,15 @@ def test_walk_workspaces_kept_are_bounded(monkeypatch):
 
     monkeypatch.setattr(ops, "_wide_workspace_cap", lambda d: 1 << 33)
     monkeypatch.setattr(ops, "_workspace", temporary)
-    monkeypatch.setattr(ops, "_slstm_workspace", lambda n, d: (temporary(n, d) and "kept", 65))
+    monkeypatch.setattr(ops, "_slstm_workspace", lambda n, d, k: (temporary(n, d) and "kept", 65))
     keep = ops._WALK_KEEP
     assert keep <= 1 << 30
-    assert ops._walk_workspace(keep, dev) == ("kept", 65)
-    assert ops._walk_workspace(keep + 1, dev) == ("own", 0)
-    assert ops._walk_workspace((1 << 33) + 1, dev) is None
+    assert ops._walk_workspace(keep, dev, (0, 0)) == ("kept", 65)
+    assert ops._walk_workspace(keep + 1, dev, (0, 0)) == ("own", 0)
+    assert ops._walk_workspace((1 << 33) + 1, dev, (0, 0)) is None
     full.append(1)
-    assert ops._walk_workspace(keep, dev) is None and ops._walk_workspace(keep + 1, dev) is None
+    assert ops._walk_workspace(keep, dev, (0, 0)) is None
+    assert ops._walk_workspace(keep + 1, dev, (0, 0)) is None
 
 
 def test_a_growing_cache_gives_its_buffer_back_first(monkeypatch):
