@@ -1555,15 +1555,16 @@ __global__ __launch_bounds__(256) void gru_rev_mfma_kernel(
 // block (X = h_prev for z and r, h_prev r for n; D the gate's pre-activation
 // gradients), so h_prev and r are read once.  4 waves; wave w owns the output
 // columns 16 w .. 16 w + 15 of each gate (four 16x16 tiles down the rows i).
-// Rows are staged through LDS 16 at a time.
+// Rows are staged through LDS 16 at a time.  r: [sequence chunk][step], a step's
+// 64 values r_row floats after those of the step before.
 constexpr int kGaRows = 16;
 constexpr int kGaPad = 80;  // fp32 LDS row stride (the 4 lane groups land on distinct banks)
 
 template <typename TX, bool PK>
 __global__ __launch_bounds__(256) void gru_ga_kernel(
-    const TX* __restrict__ h0, const TX* __restrict__ states, const float* __restrict__ gates,
-    const TX* __restrict__ g_wx, int B, int T, int H, int n_chunks, int n_split, int rows_per,
-    float* __restrict__ part, GPk pk) {
+    const TX* __restrict__ h0, const TX* __restrict__ states, const float* __restrict__ r,
+    int r_row, const TX* __restrict__ g_wx, int B, int T, int H, int n_chunks, int n_split,
+    int rows_per, float* __restrict__ part, GPk pk) {
   __shared__ float sx[2][kGaRows][kGaPad], sy[3][kGaRows][kGaPad];
   const int split = blockIdx.x % n_split;
   const int head = blockIdx.x / n_split;
@@ -1603,7 +1604,7 @@ __global__ __launch_bounds__(256) void gru_ga_kernel(
       // r stays as loaded: multiplying here would wait for these loads at
       // once instead of while the current block's products run
       st.rv =
-          *reinterpret_cast<const floatx4*>(gates + ((task * kChunk + t % kChunk) * 3 + 1) * DH + sj);
+          *reinterpret_cast<const floatx4*>(r + (task * kChunk + t % kChunk) * r_row + sj);
       st.y0 = ldr4(g_wx + wx_at(b, t, T, d, 0, head, sj));
       st.y1 = ldr4(g_wx + wx_at(b, t, T, d, 1, head, sj));
       st.y2 = ldr4(g_wx + wx_at(b, t, T, d, 2, head, sj));
@@ -1937,7 +1938,8 @@ static int run_bwd(const TX* wx, const TX* az, const TX* ar, const TX* an, const
         B, T, H, n_chunks, pk);
   PRNN_HIP(hipGetLastError());
   gru_ga_kernel<TX, PK><<<dim3(w.n_split * H), dim3(256), 0, stream>>>(
-      h0, states, w.gates, g_wx, B, T, H, n_chunks, w.n_split, w.rows_per, w.part, pk);
+      h0, states, w.gates + DH, 3 * DH, g_wx, B, T, H, n_chunks, w.n_split, w.rows_per, w.part,
+      pk);
   PRNN_HIP(hipGetLastError());
   gru_ga_reduce_kernel<<<dim3((3 * H * DH * DH + 63) / 64), dim3(256), 0, stream>>>(
       w.part, H, w.n_split, g_a);
@@ -1947,9 +1949,9 @@ static int run_bwd(const TX* wx, const TX* az, const TX* ar, const TX* an, const
 
 // The backward with the adjoint as walks over time (gru_walk.hip): no chunk
 // matrices and no carry scan, the walk forms the gates itself; then the same
-// dL/dA reduction, which reads r from the workspace.
+// dL/dA reduction, which reads r from the workspace (all that it keeps of the gates).
 struct WalkBwdWs {
-  float* gates;
+  float* r;
   float* part;
   int n_split, rows_per;
   int* hq;
@@ -1959,8 +1961,8 @@ static WalkBwdWs carve_walk_bwd(void* base, int B, int T, int H, size_t* total, 
   const int n_chunks = (T + kChunk - 1) / kChunk;
   Carver cv(base);
   WalkBwdWs w;
-  w.gates = static_cast<float*>(
-      cv.take(sizeof(float) * static_cast<size_t>(B) * H * n_chunks * kChunk * 3 * DH));
+  w.r = static_cast<float*>(
+      cv.take(sizeof(float) * static_cast<size_t>(B) * H * n_chunks * kChunk * DH));
   ga_split(B, T, H, &w.n_split, &w.rows_per);
   w.part = static_cast<float*>(
       cv.take(sizeof(float) * static_cast<size_t>(w.n_split) * 3 * H * DH * DH));
@@ -1975,12 +1977,12 @@ static int run_walk_bwd(const TX* wx, const TX* az, const TX* ar, const TX* an, 
                         int B, int T, int H, const WalkBwdWs& w, hipStream_t stream,
                         const GPk& pk) {
   const int n_chunks = (T + kChunk - 1) / kChunk;
-  gruk::launch_walk_reverse<TX>(wx, az, ar, an, h0, states, grad, g_wx, w.gates,
+  gruk::launch_walk_reverse<TX>(wx, az, ar, an, h0, states, grad, g_wx, w.r,
                                 h0 != nullptr ? g_h0 : nullptr, T, H, PK ? pk.n_seq : B, n_chunks,
                                 kChunk, PK ? pk.cu : nullptr, stream);
   PRNN_HIP(hipGetLastError());
   gru_ga_kernel<TX, PK><<<dim3(w.n_split * H), dim3(256), 0, stream>>>(
-      h0, states, w.gates, g_wx, B, T, H, n_chunks, w.n_split, w.rows_per, w.part, pk);
+      h0, states, w.r, DH, g_wx, B, T, H, n_chunks, w.n_split, w.rows_per, w.part, pk);
   PRNN_HIP(hipGetLastError());
   gru_ga_reduce_kernel<<<dim3((3 * H * DH * DH + 63) / 64), dim3(256), 0, stream>>>(
       w.part, H, w.n_split, g_a);

@@ -177,7 +177,7 @@ __device__ __forceinline__ void gate_slice(int s, const GateOps& b, GateAcc& a,
 // The adjoint walk of every (sequence, block head); see gru_walk.hip.
 template <typename TX>
 void launch_walk_reverse(const TX* wx, const TX* az, const TX* ar, const TX* an, const TX* h0,
-                         const TX* states, const TX* grad, TX* g_wx, float* gates, float* g_h0,
+                         const TX* states, const TX* grad, TX* g_wx, float* r_out, float* g_h0,
                          int T, int H, int n_rows, int n_chunks, int chunk, const int* cu,
                          hipStream_t stream);
 

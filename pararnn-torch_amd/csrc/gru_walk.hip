@@ -319,7 +319,7 @@ gruk_newton_kernel(const TX* __restrict__ wx, const TX* __restrict__ a_z,
 // (reference kernels/gru_head_factor.py:68-112).  Row i of a block is step
 // tb - i; the gates are those of the forward step at H*, made the same way.
 // Writes d_z, d_r, d_n (= dL/dwx), r in the layout the dL/dA reduction reads
-// ([sequence chunk][step][gate][channel]), and at the sequence's first step
+// ([sequence chunk][step][channel]), and at the sequence's first step
 // nu = dL/dh0.
 // ---------------------------------------------------------------------------
 struct ReverseShared {
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 gruk_reverse_kernel(const TX* __restrict__ wx, const TX* __restrict__ a_z,
                     const TX* __restrict__ a_r, const TX* __restrict__ a_n,
                     const TX* __restrict__ h0, const TX* __restrict__ states,
-                    const TX* __restrict__ grad, TX* __restrict__ g_wx, float* __restrict__ gates,
+                    const TX* __restrict__ grad, TX* __restrict__ g_wx, float* __restrict__ r_out,
                     float* __restrict__ g_h0, int T, int H, int n_chunks, int chunk,
                     const int* __restrict__ cu) {
   __shared__ ReverseShared sh;
@@ -394,7 +394,7 @@ gruk_reverse_kernel(const TX* __restrict__ wx, const TX* __restrict__ a_z,
       sh.b[to][row][l.col] = float2{r, k.d5};
       if (t >= sp.t0) {
         const size_t task = (static_cast<size_t>(sp.row) * H + head) * n_chunks + t / chunk;
-        gates[((task * chunk + t % chunk) * 3 + 1) * DH + l.col] = r;
+        r_out[(task * chunk + t % chunk) * DH + l.col] = r;
       }
     }
   };
@@ -476,11 +476,11 @@ gruk_reverse_kernel(const TX* __restrict__ wx, const TX* __restrict__ a_z,
 
 template <typename TX>
 void launch_walk_reverse(const TX* wx, const TX* az, const TX* ar, const TX* an, const TX* h0,
-                         const TX* states, const TX* grad, TX* g_wx, float* gates, float* g_h0,
+                         const TX* states, const TX* grad, TX* g_wx, float* r_out, float* g_h0,
                          int T, int H, int n_rows, int n_chunks, int chunk, const int* cu,
                          hipStream_t stream) {
   gruk_reverse_kernel<TX><<<dim3(n_rows * H), dim3(kThreads), 0, stream>>>(
-      wx, az, ar, an, h0, states, grad, g_wx, gates, g_h0, T, H, n_chunks, chunk, cu);
+      wx, az, ar, an, h0, states, grad, g_wx, r_out, g_h0, T, H, n_chunks, chunk, cu);
 }
 #define PRNN_INSTANTIATE(TX)                                                                     \
   template void launch_walk_reverse<TX>(const TX*, const TX*, const TX*, const TX*, const TX*,   \

@@ -157,3 +157,16 @@ def test_float32_warm_starts_of_a_stream_and_of_rows_have_the_same_tiles():
         rows = lib.prnn_slstm_init_workspace_size(1, T, d, P, _lib.PRNN_F32)
         assert rows > 0
         assert lib.prnn_slstm_init_packed_workspace_size(T, d, P, _lib.PRNN_F32) == rows
+
+
+def test_walk_backward_keeps_one_plane_of_gates():
+    """Of the gates the dL/dA reduction reads r alone."""
+    from pararnn_amd import _lib
+
+    if not os.path.exists(_lib.lib_path()):
+        pytest.skip("library not built (run __graft_entry__.build())")
+    lib = _lib.load()
+    plane = 4 * 256 * 2048 * 16 * 64
+    for packed in (0, 1):
+        assert plane <= lib.prnn_gru_head_walk_backward_workspace_size(256, 2048, 16, packed) \
+            < 1.2 * plane
