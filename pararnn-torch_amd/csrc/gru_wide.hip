@@ -271,9 +271,11 @@ __global__ __launch_bounds__(kThreads) void gruw_gates_kernel(
 // The gate products do not depend on the walk, so they run on other CUs and
 // leave the walk's per-step critical path with the Jacobian alone.
 //   H_{k-1} (k >= 1) and the gates pass through the workspace as tagged
-// words {value, tag}, written step by step and read with a tag check, so no
-// flag or fence orders them (the device-coherent words of the sLSTM
-// look-back); iteration 0 reads the initial guess, the last iteration writes
+// words {value, tag} and are read with a tag check, so no flag or fence orders
+// them (the device-coherent words of the sLSTM look-back).  A walk writes its
+// iterate at the end of each block, so what follows it starts on a block when
+// the walk is through with it; the gates are written as they come, z and r of
+// a block and then its n.  Iteration 0 reads the initial guess, the last iteration writes
 // `out`.  Workgroups take their (k, role, sequence, head) from a ticket in
 // start order -- iteration-major, gates before walks -- so whatever a
 // workgroup waits on belongs to a running or finished workgroup.  A wait that
@@ -335,7 +337,8 @@ __device__ __forceinline__ unsigned long long ld_word(const unsigned long long* 
 }
 
 // Where lane tid's staged values of the block at t_first live (steps clamped
-// into [t_lo, t_hi]; clamped values are never used).
+// into [t_lo, t_hi]; clamped values are never used, but waited for: the sharing
+// of gate words below counts on it).
 struct BlockAt {
   size_t row_base;
   int d;
@@ -743,10 +746,14 @@ __global__ __launch_bounds__(kThreads) void gruw_newton_kernel(
     sh.first[cx.sc] =
         (cx.live && h0 != nullptr) ? h0[static_cast<size_t>(cx.sp.seq) * cx.d + cx.col] : 0.f;
   if (cx.sp.t0 >= cx.sp.t1) return;
-  // Iterations k and k + 2 share gate words: the gate workgroups of k + 2
-  // reach block b only after the iterate of k + 1 covers it, i.e. after the
-  // walk of k has finished block b and so read its gates for the last time
-  // (distinct tags keep the two iterations' words apart).
+  // Iterations k and k + 2 share gate words (distinct tags keep them apart).
+  // No word is overwritten before its last read: the gates of a block b of any
+  // iteration wait for at least one step of b of the iterate before (the rows
+  // b - 1 + s of its steps, and in a partly filled block, even of one step, the
+  // clamped rows behind them, which are its last step), and a walk writes that
+  // only at the end of b, when it has the gates of b in LDS.  So gates k + 2 of
+  // b follow walk k + 1 through b, which needs gates k + 1 of b, which follow
+  // walk k through b.
   unsigned long long* gk = gates + static_cast<size_t>(k % 2) * 3 * cx.btd;
   const NewtonSrc<TX> src{wx,    gk,    cx.btd, tag_base + 1 + k, guess,
                           k == 0 ? nullptr : iters + (k - 1) * cx.btd, tag_base + k};
