@@ -93,3 +93,27 @@ def test_captured_replays_and_an_input_that_is_the_state():
         own = state.clone()
         D.decode_step(cell, own, own, out=own)
         assert torch.equal(own, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_route_at_the_line(dtype, monkeypatch):
+    """The rule as it stands, on either side of its line: one row below it (and on it)
+    the kernel projects, one row above it the library; same step."""
+    d_in = 1024
+    rows = (1 << (26 if dtype is torch.bfloat16 else 24)) // (d_in * d_in)
+    took = []
+    launch = D._launch
+    monkeypatch.setattr(D, "_launch", lambda *a: (took.append(a[5]), launch(*a))[1])
+    for B, projects in ((rows - 1, True), (rows, True), (rows + 1, False)):
+        g = torch.Generator().manual_seed(B)
+        cell = ParaSLSTM(d_in, d_in).to(DEV, dtype)
+        with torch.no_grad():
+            w = torch.zeros(4 * d_in, d_in)
+            w[:, :32] = torch.randint(-1, 2, (4 * d_in, 32), generator=g) / 4
+            cell.W_x.weight.copy_(w)
+            x = (torch.randint(-1, 2, (B, d_in), generator=g) / 4).to(DEV, dtype)
+            state = torch.rand(B, 4, d_in, generator=g).to(DEV, dtype)
+            want = D.decode_step(cell, state, wx=cell.W_x(x))
+            got = D.decode_step(cell, state, x)
+        assert (took[-1] is cell.W_x) is projects
+        assert torch.equal(got, want)

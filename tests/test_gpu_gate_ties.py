@@ -1,8 +1,8 @@
 """The gate split of the sLSTM Newton kernels at and next to ties.
 
 One Newton iteration on steps whose left = z_f + m and z_i are equal (the max's
-derivative is split 0.5 / 0.5), one float apart, 1e-30 apart, or
-infinite apart, in fp32, against the cell's own step and Jacobian in float64: an
+derivative is split 0.5 / 0.5), one float apart, 1e-30 apart, or up
+to 60 apart (the smaller gate, e^-60, is nothing beside the larger), in fp32, against the cell's own step and Jacobian in float64: an
 iteration is H + delta with delta_t = J_t delta_{t-1} + F_t, so with T = 2 steps the
 second one shows J.  Tolerance: 40 operations of relative error 2^-23 on terms
 of at most 8 in size (each derivative is at most 4, delta at most 2)."""
