@@ -296,10 +296,8 @@ static int run_init(const TX* wx, const TX* r, const TX* h0, TX* states, int B, 
     if (pk.cu != nullptr) {
       launch_picard_packed(wx, r, h0, states, T, d, P, eps, w.lb, w.hlast, stream, pk);
     } else if constexpr (sizeof(TX) == 4) {
-      if (deterministic())
-        PRNN_LAUNCH(kPicardF32.L, kPicardF32.W, 2, true);
-      else
-        PRNN_LAUNCH(kPicardF32.L, kPicardF32.W, 2, false);
+      // the deterministic walk always (see kPicardF32)
+      PRNN_LAUNCH(kPicardF32.L, kPicardF32.W, 2, true);
     } else {
       if (deterministic()) PRNN_LAUNCH(24, 4, 3, true);
       else if constexpr (std::is_same<TX, f16>::value) PRNN_LAUNCH(24, 4, 3, false);

@@ -1384,10 +1384,18 @@ constexpr Shape kNewtonGuessDefault{24, 4};
 constexpr Shape kNewtonWorkDefault{24, 4};
 constexpr Shape kNewtonF32{16, 8};
 constexpr Shape kPicardDefault{24, 4};
-// fp32, all six passes of P = 5 at d=512, B=8, T=16384: 0.86 ms (32x4, two waves
-// per SIMD, no spills) against 0.85 (20x4), 0.90 (16x4), 0.95 (12x4, 24x4) and
-// 2.18 ms as one launch per pass; at d=256, B=1, T=131072 0.58 against 0.63
-// (20x4) and 1.31 ms; at d=256, B=8, T=2048, P=3 84 against 93 and 142 us.
+// fp32, all six passes of P = 5 at d=512, B=8, T=16384 under the default walk:
+// 0.83 ms (32x4, two waves per SIMD, no spills) against 0.85 (20x4), 0.90 (16x4),
+// 0.95 (12x4, 24x4) and 2.12 ms as one launch per pass.
+//
+// fp32 warm starts, rectangular and packed, always take the deterministic walk.  What
+// they are off by Newton at a pinned K amplifies (a sequence of 4096 steps, K = P = 3:
+// 7e-6 of n, 8e-5 after), and with all passes in flight at once the default walk's
+// order of sums varied more from run to run than with a launch per pass: after Newton
+// 6.7e-5 .. 8.7e-5, against 6.3e-5 .. 7.7e-5 then and 8.0e-5 every time now.  It costs
+// 0.83 -> 0.91 ms there, 0.55 -> 0.61 at d=256, B=1, T=131072 (1.27 with a launch per
+// pass), 60 -> 63 us at d=256, B=8, T=2048, P=3 (121), and in packed streams 0.34 ->
+// 0.38 ms at N=16019, d=860, 95 sequences (0.69).
 constexpr Shape kPicardF32{32, 4};
 constexpr Shape kNewtonFusedDefault{20, 4};
 constexpr Shape kNewtonFusedF32{16, 4};
@@ -1397,9 +1405,8 @@ constexpr Shape kNewtonFusedF32{16, 4};
 // loop: no spills); the single-iteration launches run shorter tiles.
 constexpr Shape kPicardPacked{24, 4};
 // the rectangular launch's tile: a stream and the same sequences as padded rows
-// then compose their carries alike.  With 28 steps (no spills, against 7 registers
-// here: N=16019, d=860, 95 sequences 0.36 against 0.375 ms, one launch per pass
-// 0.75) the gradients of the two differed by twice as much.
+// then compose their carries alike.  With 28 steps (which do not spill; 32 spill 7
+// registers, 4% of the launch) the gradients of the two differed by twice as much.
 constexpr Shape kPicardPackedF32 = kPicardF32;
 inline Shape picard_packed_shape(bool narrow) { return narrow ? kPicardPacked : kPicardPackedF32; }
 constexpr Shape kNewtonFusedPacked{20, 4};

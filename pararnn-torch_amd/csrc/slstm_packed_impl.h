@@ -22,10 +22,15 @@ void launch_picard_packed(const TN* wx, const TN* r, const TN* h0, TN* out, int 
       <<<dim3(g.n_tiles), dim3(64 * sh.W), 0, stream>>>(                                        \
       wx, r, h0, out, 1, T, d, g.n_cb, g.n_tiles, P, eps, lb.counters + 1, lb.agg, lb.incl,   \
       hlast, lb.tag_base, lb.spin(), pk)
-  if (deterministic())
+  // fp32: the deterministic walk always (see kPicardF32)
+  if constexpr (sizeof(TN) == 4) {
     PRNN_LAUNCH(true);
-  else
-    PRNN_LAUNCH(false);
+  } else {
+    if (deterministic())
+      PRNN_LAUNCH(true);
+    else
+      PRNN_LAUNCH(false);
+  }
 #undef PRNN_LAUNCH
 }
 

@@ -80,3 +80,23 @@ def test_packed(lengths, P):
         a, b = int(cu[s]), int(cu[s + 1])
         want = _walk(wx[:, a:b].double(), r.double(), h0[s:s + 1].double(), P)
         _check(got[:, a:b], want, b - a, P)
+
+
+@pytest.mark.parametrize("lengths", [[4096] + [17] * 40, [2500, 31, 900, 700, 12, 60], None])
+def test_repeats_bit_for_bit(lengths):
+    """float32 warm starts do not depend on the order in which tiles finish."""
+    d, B, N = (64, 1, sum(lengths)) if lengths else (200, 3, 4097)
+    g = torch.Generator().manual_seed(N)
+    wx = torch.randn(B, N, 4 * d, generator=g).to(DEV)
+    r = (torch.randn(4, d, generator=g) * 0.3).to(DEV)
+    h0 = torch.rand(len(lengths) if lengths else B, 4, d, generator=g).to(DEV)
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()]).to(DEV) if lengths else None
+    print(f"case repeats B={B} N={N} packed={lengths is not None}", flush=True)
+    outs = [ops.slstm_init_fused(wx, r, h0, cu, picard_iters=3, eps=EPS) for _ in range(30)]
+    prev = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(True, warn_only=True)
+    try:
+        outs.append(ops.slstm_init_fused(wx, r, h0, cu, picard_iters=3, eps=EPS))
+    finally:
+        torch.use_deterministic_algorithms(prev)
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
