@@ -9,8 +9,8 @@ On this path the flag also switches the HIP library's look-back scans into
 their deterministic mode (``prnn_set_deterministic``, set before each sLSTM
 launch): every tile's carry is then the serial chain of published tile
 aggregates, so forward states, ``grad_x``/``grad_h0`` and the parameter
-gradients are bit-identical between runs.  The head GRU scans are
-deterministic in either mode, and every reduction (R, A, bias, the split-K
+gradients are bit-identical between runs.  The head GRU scans and the float32
+warm starts are deterministic in either mode, and every reduction (R, A, bias, the split-K
 ``W_x`` partials) sums in a fixed order with no atomics.  The reference's
 ``CUBLAS_WORKSPACE_CONFIG`` advice (determinism.py:48-61) concerns cuBLAS
 workspaces and has no counterpart on ROCm's GEMM path.
