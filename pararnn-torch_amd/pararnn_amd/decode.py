@@ -160,8 +160,11 @@ def _projects(proj: nn.Module | None, rows: Tensor, d: int, gates: int, fused: b
     tensor subclasses, modes, autocast, tracing), on rows that it can read as they
     are.  ``out`` must not overlap ``rows``: the projection is still being read when
     the first channels of the next state are written."""
-    size = rows.element_size()
-    if type(proj) is not nn.Linear or not _small_step(rows.shape[0], d, rows.shape[1], size, fused):
+    (batch, k), size = rows.shape, rows.element_size()
+    # what keeps the library call by its sizes is told first: live steps are bound by
+    # the host, and the whole list takes 3 us of 37
+    if (k * size % 16 or not _small_step(batch, d, k, size, fused)
+            or type(proj) is not nn.Linear):
         return False
     if (proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks
             or proj._backward_pre_hooks or "forward" in proj.__dict__
@@ -174,13 +177,13 @@ def _projects(proj: nn.Module | None, rows: Tensor, d: int, gates: int, fused: b
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()):
         return False
     dtype, dev = rows.dtype, rows.device
-    if w.dtype != dtype or w.device != dev or w.shape != (gates * d, rows.shape[1]):
+    if w.dtype != dtype or w.device != dev or w.shape != (gates * d, k):
         return False
     if bias is not None and (bias.dtype != dtype or bias.device != dev
                              or not bias.is_contiguous()):
         return False
     x0, w0, o0 = rows.data_ptr(), w.data_ptr(), out.data_ptr()
-    if (x0 | w0 | rows.shape[1] * size) % 16 or not rows.is_contiguous() or not w.is_contiguous():
+    if (x0 | w0) % 16 or not rows.is_contiguous() or not w.is_contiguous():
         return False
     return (not rows.is_neg() and not w.is_neg() and rows.numel() > 0
             and (x0 + rows.numel() * size <= o0 or o0 + out.numel() * out.element_size() <= x0))
@@ -215,12 +218,16 @@ def _launch(cell: nn.Module, kind: str, state: Tensor, gates: Tensor, tgt: _Targ
     clamp = (0.0, 0) if cap is None else (float(cap), 1)
     table = None if tgt.table is None else _ptr(tgt.table)
     # the leading operands of either entry
-    src = (_ptr(gates),) if proj is None else (_ptr(gates), _ptr(proj.weight), _ptr(proj.bias))
-    d_in = () if proj is None else (int(gates.shape[1]),)
+    if proj is None:
+        src, d_in = (_ptr(gates),), ()
+    else:
+        src, d_in = (_ptr(gates), _ptr(proj.weight), _ptr(proj.bias)), (int(gates.shape[1]),)
     if kind == "slstm":
         if proj is None and gates.shape[-1] != 4 * d:
             raise ValueError(f"ParaSLSTM wx last dim {gates.shape[-1]} != 4 * d_h={4 * d}")
-        r = cell.R if cell.R.is_contiguous() else cell.R.contiguous()
+        r = cell.R
+        if not r.is_contiguous():
+            r = r.contiguous()
         code = _validate("decode_slstm", state, gates, r, tgt.out)
         with torch.cuda.device(state.device):
             entry = lib.prnn_slstm_decode if proj is None else lib.prnn_slstm_decode_x
@@ -268,12 +275,11 @@ def decode_step(cell: nn.Module, state: Tensor, x: Tensor | None = None, *,
     if wx is None:
         gates = _one_step(x, "x")
         linear = getattr(cell, "W_x", None)
-        dest = out if out is not None else state
         if _projects(linear, gates, int(cell.d_h), 4 if kind == "slstm" else 3,
-                     cell.mix == "diag", dest):
+                     cell.mix == "diag", state if out is None else out):
             proj = linear
         else:
-            gates = decode_wx(cell, x)
+            gates = decode_wx(cell, gates) if linear is None else linear(gates)
     else:
         gates = _one_step(wx, "wx")
     gates = _laid_out(gates, "wx", capturing)

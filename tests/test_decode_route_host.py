@@ -100,3 +100,18 @@ def test_large_steps_keep_the_library():
     assert D._small_step(64, 1024, 1024, 2, True) and not D._small_step(128, 1024, 1024, 2, True)
     assert D._small_step(16, 1024, 1024, 4, True) and not D._small_step(16, 1024, 1024, 4, False)
     assert D._small_step(512, 64, 64, 4, False) and not D._small_step(64, 1024, 1024, 4, True)
+
+
+@pytest.mark.parametrize("d_in,rows,dtype", [(6, 2, torch.float32), (555, 3, torch.bfloat16),
+                                             (1024, 4096, torch.float32)])
+def test_sizes_are_told_before_anything_is_looked_at(d_in, rows, dtype, monkeypatch):
+    """Rows of a partial 16-byte word and large steps keep the library call without the
+    cost of the other checks."""
+    def looked(*a, **k):
+        raise AssertionError("looked further")
+
+    monkeypatch.setattr(torch, "is_autocast_enabled", looked)
+    monkeypatch.setattr(nn.modules.module, "_has_any_global_hook", looked)
+    lin = nn.Linear(d_in, 64).to(dtype)
+    assert not D._projects(lin, torch.zeros(rows, d_in, dtype=dtype), 16 if d_in < 1024 else 1024,
+                           4, True, torch.zeros(1))
