@@ -78,6 +78,7 @@ _stream_locks = tuple(threading.RLock() for _ in range(16))
 
 
 def _stream_key(dev: torch.device) -> tuple[int, int]:
+    """The current stream: (device index, stream handle)."""
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     return index, torch.cuda.current_stream(dev).cuda_stream
 
@@ -230,7 +231,7 @@ def slstm_init_fused(
             ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_init_ex(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(out), batch, time, d_h, int(picard_iters),
-                float(eps), code, _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                float(eps), code, _ptr(ws), ws.numel(), tag, key[1],
             )
         else:
             nbytes = lib.prnn_slstm_init_packed_workspace_size(time, d_h, picard_iters, code)
@@ -238,7 +239,7 @@ def slstm_init_fused(
             rc = lib.prnn_slstm_init_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(out), time, d_h, int(picard_iters),
                 float(eps), code, _ptr(cs32), n_seq, _ptr(bt), _ptr(ws), ws.numel(), tag,
-                _stream(wx.device),
+                key[1],
             )
     _lib.check(rc, "slstm_init_fused")
     _check_lookback(ws, "slstm_init_fused")
@@ -320,7 +321,7 @@ def newton_slstm_fused(
             rc = lib.prnn_slstm_newton_ex(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), batch, time, d_h,
                 int(max_iters), float(omega), float(eps), code, _ptr(ws), ws.numel(), tag,
-                _stream(wx.device),
+                key[1],
             )
         else:
             nbytes = lib.prnn_slstm_newton_packed_workspace_size(time, d_h, int(max_iters), code)
@@ -328,7 +329,7 @@ def newton_slstm_fused(
             rc = lib.prnn_slstm_newton_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), time, d_h,
                 int(max_iters), float(omega), float(eps), code, _ptr(cs32), n_seq, _ptr(bt),
-                _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                _ptr(ws), ws.numel(), tag, key[1],
             )
     _lib.check(rc, "newton_slstm_fused")
     _check_lookback(ws, "newton_slstm_fused")
@@ -366,7 +367,7 @@ def slstm_newton_step(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor, 
             rc = lib.prnn_slstm_newton_step(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), int(in_f32), _ptr(out), batch, time,
                 d_h, float(omega), float(eps), code, _ptr(ws), ws.numel(), tag,
-                _stream(wx.device),
+                key[1],
             )
         else:
             nbytes = lib.prnn_slstm_newton_packed_workspace_size(time, d_h, 1, code)
@@ -374,7 +375,7 @@ def slstm_newton_step(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor, 
             rc = lib.prnn_slstm_newton_step_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), int(in_f32), _ptr(out), time, d_h,
                 float(omega), float(eps), code, _ptr(cs32), n_seq, _ptr(bt), _ptr(ws),
-                ws.numel(), tag, _stream(wx.device),
+                ws.numel(), tag, key[1],
             )
     _lib.check(rc, "slstm_newton_step")
     _check_lookback(ws, "slstm_newton_step")
@@ -408,7 +409,7 @@ def slstm_newton_eager(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor,
             ws, tag = _slstm_workspace(nbytes, wx.device, key)
             rc = lib.prnn_slstm_newton_eager(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), batch, time, d_h,
-                float(omega), float(eps), code, _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                float(omega), float(eps), code, _ptr(ws), ws.numel(), tag, key[1],
             )
         else:
             nbytes = lib.prnn_slstm_newton_packed_workspace_size(time, d_h, 1, code)
@@ -416,7 +417,7 @@ def slstm_newton_eager(wx: Tensor, r: Tensor, h0: Tensor | None, states: Tensor,
             rc = lib.prnn_slstm_newton_eager_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(out), time, d_h, float(omega),
                 float(eps), code, _ptr(cs32), n_seq, _ptr(bt), _ptr(ws), ws.numel(), tag,
-                _stream(wx.device),
+                key[1],
             )
     _lib.check(rc, "slstm_newton_eager")
     _check_lookback(ws, "slstm_newton_eager")
@@ -473,13 +474,13 @@ def slstm_backward_fused(
             rc = lib.prnn_slstm_backward_ex(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(grad), _ptr(g_wx), _ptr(g_r),
                 _ptr(g_h0), _ptr(g_b), batch, time, d_h, float(eps), code, _ptr(ws), ws.numel(),
-                tag, _stream(wx.device),
+                tag, key[1],
             )
         else:
             rc = lib.prnn_slstm_backward_packed(
                 _ptr(wx), _ptr(r), _ptr(h0), _ptr(states), _ptr(grad), _ptr(g_wx), _ptr(g_r),
                 _ptr(g_h0), _ptr(g_b), time, d_h, float(eps), code, _ptr(cs32), n_seq,
-                _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                _ptr(ws), ws.numel(), tag, key[1],
             )
     _lib.check(rc, "slstm_backward_fused")
     _check_lookback(ws, "slstm_backward_fused")
@@ -765,7 +766,7 @@ def _gru_head_dense(wx, a_z, a_r, a_n, h0, max_iters, omega, cs=None):
                 rc = lib.prnn_gru_head_walk_newton(
                     _ptr(wx), _ptr(a_z), _ptr(a_r), _ptr(a_n), _ptr(h0), _ptr(out), batch, time,
                     hb.n_blocks, int(max_iters), float(omega), code, _ptr(cs32),
-                    0 if cs is None else rows, _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                    0 if cs is None else rows, _ptr(ws), ws.numel(), tag, key[1],
                 )
         if held is not None:
             _lib.check(rc, "newton_gru_head_fused")
@@ -1013,7 +1014,7 @@ def _gru_head_wide(wx, a_z, a_r, a_n, h0, max_iters, omega, code, cs=None):
             rc = lib.prnn_gru_wide_newton(
                 _ptr(wx_c), _ptr(a_k[0]), _ptr(a_k[1]), _ptr(a_k[2]), _ptr(h0_c), _ptr(guess),
                 _ptr(out), batch, time, n_heads, d_head, max_iters, float(omega), code,
-                _ptr(cs32), n_seq, _ptr(ws), ws.numel(), tag, _stream(wx.device),
+                _ptr(cs32), n_seq, _ptr(ws), ws.numel(), tag, key[1],
             )
         _lib.check(rc, "newton_gru_head_fused (wide heads)")
         _check_lookback(ws, "newton_gru_head_fused (wide heads)")
